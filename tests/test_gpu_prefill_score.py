@@ -68,3 +68,38 @@ def test_prefill_block_mass_agrees_with_compute_block_scores(device):
     ref = engine.compute_block_scores(probs)
     got = kernels.prefill_block_mass(q, k, 16, D ** -0.5)[0]
     torch.testing.assert_close(got, ref, rtol=1e-4, atol=1e-8)
+
+
+@pytest.mark.parametrize("B,H,Hkv,T,D,dtype", [
+    (1, 1, 1, 2048, 64, torch.float16),      # one head per workgroup; the last length with four waves
+    (1, 2, 1, 2049, 64, torch.bfloat16),     # two heads; the first with eight
+    (1, 3, 1, 1000, 128, torch.float16),     # an idle slot
+    (1, 5, 1, 530, 128, torch.bfloat16),     # two head sets, the second with three idle slots
+    (1, 2, 2, 4096, 64, torch.float16),      # the last one-pass length
+    (1, 2, 1, 4100, 64, torch.float16),      # two passes, partial last tile
+    (9, 1, 1, 65, 128, torch.float16),       # pairs not a multiple of the XCDs, one row past a 64-query block
+])
+def test_prefill_block_mass_edges(device, B, H, Hkv, T, D, dtype):
+    print(f"[prefill-edge] B={B} H={H} Hkv={Hkv} T={T} D={D} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(T + H)
+    q = torch.randn((B, H, T, D), generator=g).to(dtype)
+    k = torch.randn((B, Hkv, T, D), generator=g).to(dtype)
+    got = kernels.prefill_block_mass(q.to(device), k.to(device), 16, D ** -0.5).cpu().numpy()
+    want = oracle_mass(q.float().numpy(), k.float().numpy(), D ** -0.5, 16)
+    np.testing.assert_allclose(got, want, rtol=1e-4, atol=1e-9)
+
+
+@pytest.mark.parametrize("T,growth", [(700, 30.0), (700, -30.0), (4200, 30.0)])
+def test_prefill_block_mass_growing_logits(device, T, growth):
+    """Logits that grow along the prompt by far more than 2^64 in probability
+    (the rows' references are raised and their earlier sums rescaled), or
+    fall (later sums are tiny).  Logits reach about |growth| * 10 in log2
+    units: a few fp32 roundings of 300 * 2^-24 in the exponent are 1e-4
+    relative, so the bound is 5e-4."""
+    g = torch.Generator().manual_seed(5)
+    ramp = torch.linspace(0.1, 1.0, T) if growth > 0 else torch.linspace(1.0, 0.1, T)
+    q = torch.randn((1, 4, T, 64), generator=g).half()
+    k = (torch.randn((1, 1, T, 64), generator=g) * (ramp * abs(growth))[None, None, :, None]).half()
+    got = kernels.prefill_block_mass(q.to(device), k.to(device), 16, 64 ** -0.5).cpu().numpy()
+    want = oracle_mass(q.float().numpy(), k.float().numpy(), 64 ** -0.5, 16)
+    np.testing.assert_allclose(got, want, rtol=5e-4, atol=1e-9)
