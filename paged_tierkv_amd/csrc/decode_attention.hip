@@ -686,7 +686,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
     const int32_t* __restrict__ a_seq_nblocks, int32_t a_stride, int32_t a_num_blocks,
     int32_t a_kvh_splits, uint32_t a_split_magic, DecodeParams p) {
   constexpr int DS = D / 16;
-  extern __shared__ float s_dyn[];               // [NW][G][D] wave accumulators, then the LDS stage
+  extern __shared__ __align__(16) float s_dyn[];   // [NW][G][D] wave accumulators, then the LDS stage
   __shared__ int4 s_list[MAX_LIST];              // (block, slot, len, state)
   __shared__ int s_wcnt[2][PRE_CHUNKS * MAX_WAVES];   // per (chunk, wave): HOT / WARM counts
   __shared__ int s_wcold[MAX_WAVES];
@@ -1070,8 +1070,8 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
         qsum += half_lo(h2) + half_hi(h2);
       }
     }
-    qsum += shfl_xor_f(qsum, 16);
-    qsum += shfl_xor_f(qsum, 32);
+    qsum += xor16_f(qsum);
+    qsum += xor32_f(qsum);
   }
 
   // ---- per-wave tile loops -------------------------------------------------
@@ -1212,11 +1212,23 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
   if (bad) atomicOr(p.ws_err, bad);
 
   // ---- merge the waves in LDS (one barrier) ----------------------------------
-  float l = st.l_part + shfl_xor_f(st.l_part, 16);
-  l += shfl_xor_f(l, 32);
-  float corr = st.corr + shfl_xor_f(st.corr, 16);
-  corr += shfl_xor_f(corr, 32) + st.ocorr;
+  float l = st.l_part + xor16_f(st.l_part);
+  l += xor32_f(l);
+  float corr = st.corr + xor16_f(st.corr);
+  corr += xor32_f(corr) + st.ocorr;
+  // A head's row of the merge buffer holds its dims in runs of DS floats (one
+  // run per accumulator register index r and lane group g: dims
+  // (4g + r) * DS ..), stored as 16-byte vectors at run position
+  // 4r + (g + head) % 4: the four groups of one r are neighbours and the
+  // heads are rotated, so a store's lanes spread over the banks.  (In dim
+  // order, as scalar stores, the 16 storing lanes of a wave fell on two
+  // banks: 1.9 us from the last tile to the barrier with eight waves of one
+  // tile each, 0.9 now.)
   float* s_acc = s_dyn;   // [nw][G][D]
+  auto dim_of = [](int h, int pos) -> int {
+    const int run = pos / DS;
+    return (4 * (((run & 3) - h) & 3) + (run >> 2)) * DS + pos % DS;
+  };
   if (head_ok) {
     if (g == 0) {
       s_m[w][n] = st.m_run;
@@ -1225,7 +1237,9 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int s = 0; s < DS; ++s) s_acc[(w * G + n) * D + (4 * g + r) * DS + s] = st.acc[s][r] - corr;
+      for (int s = 0; s < DS; s += 4)
+        *reinterpret_cast<f32x4*>(s_acc + (w * G + n) * D + (4 * r + ((g + n) & 3)) * DS + s) =
+            f32x4{st.acc[s][r] - corr, st.acc[s + 1][r] - corr, st.acc[s + 2][r] - corr, st.acc[s + 3][r] - corr};
   }
   if constexpr (SCORES) {
     // The first pass's blanks into the LDS block stage.
@@ -1352,7 +1366,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
       wave_ml(h, M, L, fw);
       const float A = wave_acc(i, fw);
       cold_adjust<COLD_ZERO>(M, L, f, cold_tokens);
-      out[i] = from_f32<QT>((L > 0.f) ? A * f / (L * PBOOST) : 0.f);
+      out[h * D + dim_of(h, i - h * D)] = from_f32<QT>((L > 0.f) ? A * f / (L * PBOOST) : 0.f);
     }
     if (SCORES && stage_mode == STAGE_LDS_BLOCK) finalize_scores();
     if (SCORES && stage_mode == STAGE_GLOBAL) flush_blanks(false);
@@ -1441,7 +1455,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
     }
     float f;
     cold_adjust<COLD_ZERO>(M, L, f, cold_tokens);
-    out[i] = from_f32<QT>((L > 0.f) ? A * f / (L * PBOOST) : 0.f);
+    out[h * D + dim_of(h, d)] = from_f32<QT>((L > 0.f) ? A * f / (L * PBOOST) : 0.f);
   }
   flush_stage();
 }
