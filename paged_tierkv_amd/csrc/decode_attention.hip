@@ -6,9 +6,9 @@
 //
 // Fast path (block_size 16, head_dim 64 or 128, GQA group <= 16), one kernel
 // (a second one finalises the score sums of split launches):
-//   * workgroup = (sequence, kv head, split), 8 waves (4 when the GQA group
-//     exceeds 8); the whole GQA group is served by one pass over each K/V
-//     byte; unsplit launches of a batch that is a multiple of 8 place each
+//   * workgroup = (sequence, kv head, split), 4 or 8 waves (plan_cost; 4 when
+//     the GQA group exceeds 8); the whole GQA group is served by one pass over
+//     each K/V byte; unsplit launches of a batch that is a multiple of 8 place each
 //     sequence's kv heads on one XCD;
 //   * every workgroup scans its sequence's table row and keeps its share of
 //     the resident blocks, HOT and WARM ranked separately: a contiguous range
@@ -140,6 +140,16 @@ __device__ __forceinline__ void store_dev(float* p, float v) {
 }
 __device__ __forceinline__ float load_dev(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Two neighbouring values (8-byte aligned) in one access of either kind.
+__device__ __forceinline__ void store_dev2(float* p, float a, float b) {
+  const uint64_t v = uint64_t(__float_as_uint(a)) | (uint64_t(__float_as_uint(b)) << 32);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_dev2(const float* p, float& a, float& b) {
+  const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  a = __uint_as_float(uint32_t(v));
+  b = __uint_as_float(uint32_t(v >> 32));
 }
 // Workgroup barrier that orders LDS accesses only.  __syncthreads() also
 // waits for the wave's outstanding global stores (on gfx9 they count in the
@@ -672,10 +682,11 @@ __device__ __forceinline__ float block_score(float2 e, float M, float inv_l, flo
 // Score reduction tree of a head's row: `parts` contiguous ranges of
 // ceil(nb / parts) blocks, one wave each (lane l folds blocks lo + l,
 // lo + l + 64, ... with fold_round, then wave_combine_ms), the parts
-// combined in ascending order.  parts = nw / G when the unit's G heads fit
-// in its nw waves, else 1; the decode workgroup and the finalisation kernel
-// both follow it, so score sums do not depend on the launch's split count.
-__host__ __device__ inline int score_parts(int groups, int nw) { return groups <= nw ? nw / groups : 1; }
+// combined in ascending order.  parts = 8 / G up to eight heads, else 1: a
+// function of the GQA group alone.  The decode workgroup and the finalisation
+// kernel both follow it, so score sums do not depend on the launch's split
+// and wave counts.
+__host__ __device__ inline int score_parts(int groups) { return groups <= 8 ? 8 / groups : 1; }
 
 // The arguments the list build needs first come ahead of the parameter block
 // so that they can be preloaded into scalar registers at wave launch.
@@ -1294,7 +1305,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
   // LDS only, so that no wave waits there for its output stores.
   auto finalize_scores = [&]() {
     const int stride = int(p.table_stride);
-    const int parts = score_parts(G, nw);
+    const int parts = score_parts(G);
     const int ntask = G * parts;
     const int chunk = (nb + parts - 1) / parts;
     auto entry = [&](int h, int blk) -> float2 {
@@ -1380,10 +1391,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
     wave_ml(h, M, L, fw);
     const int64_t pi = (int64_t(unit) * splits + split) * G + h;
     store_dev(p.ws_acc + pi * D + (i - h * D), wave_acc(i, fw));
-    if (i - h * D == 0) {
-      store_dev(p.ws_ml + pi * 2 + 0, M);
-      store_dev(p.ws_ml + pi * 2 + 1, L);
-    }
+    if (i - h * D == 0) store_dev2(p.ws_ml + pi * 2, M, L);
   }
   // Every wave's device-coherent stores complete before the arrival is counted.
   __builtin_amdgcn_s_waitcnt(0);
@@ -1419,44 +1427,68 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
     return;
   }
   // Log-sum-exp merge of the splits' partials (tierkv_triton.py:231-264).
-  // Each output element loads every split's (m, l, acc) at once (MERGE_UNROLL
-  // splits per round trip) and merges them in registers.
-  for (int i = tid; i < G * D; i += nthreads) {
-    const int h = i / D;
-    const int d = i - h * D;
-    float M = -INFINITY, L = 0.f, A = 0.f;
-    for (int sp0 = 0; sp0 < splits; sp0 += MERGE_UNROLL) {
-      float av[MERGE_UNROLL], mv[MERGE_UNROLL], lv[MERGE_UNROLL];
+  // Every output element loads all splits' (m, l) and acc at once
+  // (MERGE_UNROLL splits per round trip) and merges them in registers.  When
+  // the unit has more elements than the workgroup threads, a thread takes two
+  // at a time, so that four waves merge a group of four heads in one round
+  // trip (64 units of 256 blocks in 4 splits: 17.2 -> 16.6 us; two at a time
+  // with eight waves, where the second is idle, cost 0.6).
+  auto merge = [&](auto E_) {
+    constexpr int E = decltype(E_)::value;
+    for (int i0 = tid; i0 < G * D; i0 += E * nthreads) {
+      int hh[E], dd[E];
+      float M[E], L[E], A[E];
 #pragma unroll
-      for (int k = 0; k < MERGE_UNROLL; ++k) {
-        const int64_t pi = (int64_t(unit) * splits + min(sp0 + k, splits - 1)) * G + h;
-        av[k] = load_dev(p.ws_acc + pi * D + d);
-        mv[k] = load_dev(p.ws_ml + pi * 2);
-        lv[k] = load_dev(p.ws_ml + pi * 2 + 1);
+      for (int e = 0; e < E; ++e) {
+        const int i = min(i0 + e * nthreads, G * D - 1);
+        hh[e] = i / D;
+        dd[e] = i - hh[e] * D;
+        M[e] = -INFINITY;
+        L[e] = A[e] = 0.f;
       }
-      float Mn = M;
+      for (int sp0 = 0; sp0 < splits; sp0 += MERGE_UNROLL) {
+        float av[E][MERGE_UNROLL], mv[E][MERGE_UNROLL], lv[E][MERGE_UNROLL];
 #pragma unroll
-      for (int k = 0; k < MERGE_UNROLL; ++k)
-        if (sp0 + k < splits) Mn = fmaxf(Mn, mv[k]);
-      if (Mn != -INFINITY) {
-        const float rescale = (M == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
-        A *= rescale;
-        L *= rescale;
+        for (int e = 0; e < E; ++e)
 #pragma unroll
-        for (int k = 0; k < MERGE_UNROLL; ++k) {
-          if (sp0 + k < splits && mv[k] != -INFINITY) {
-            const float wgt = __builtin_amdgcn_exp2f(mv[k] - Mn);
-            A += av[k] * wgt;
-            L += lv[k] * wgt;
+          for (int k = 0; k < MERGE_UNROLL; ++k) {
+            const int64_t pi = (int64_t(unit) * splits + min(sp0 + k, splits - 1)) * G + hh[e];
+            av[e][k] = load_dev(p.ws_acc + pi * D + dd[e]);
+            load_dev2(p.ws_ml + pi * 2, mv[e][k], lv[e][k]);
+          }
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          float Mn = M[e];
+#pragma unroll
+          for (int k = 0; k < MERGE_UNROLL; ++k)
+            if (sp0 + k < splits) Mn = fmaxf(Mn, mv[e][k]);
+          if (Mn != -INFINITY) {
+            const float rescale = (M[e] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M[e] - Mn);
+            A[e] *= rescale;
+            L[e] *= rescale;
+#pragma unroll
+            for (int k = 0; k < MERGE_UNROLL; ++k) {
+              if (sp0 + k < splits && mv[e][k] != -INFINITY) {
+                const float wgt = __builtin_amdgcn_exp2f(mv[e][k] - Mn);
+                A[e] += av[e][k] * wgt;
+                L[e] += lv[e][k] * wgt;
+              }
+            }
+            M[e] = Mn;
           }
         }
-        M = Mn;
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        if (i0 + e * nthreads >= G * D) continue;
+        float f;
+        cold_adjust<COLD_ZERO>(M[e], L[e], f, cold_tokens);
+        out[hh[e] * D + dim_of(hh[e], dd[e])] = from_f32<QT>((L[e] > 0.f) ? A[e] * f / (L[e] * PBOOST) : 0.f);
       }
     }
-    float f;
-    cold_adjust<COLD_ZERO>(M, L, f, cold_tokens);
-    out[h * D + dim_of(h, d)] = from_f32<QT>((L > 0.f) ? A * f / (L * PBOOST) : 0.f);
-  }
+  };
+  if (G * D > nthreads) merge(std::integral_constant<int, 2>{});
+  else merge(std::integral_constant<int, 1>{});
   flush_stage();
 }
 
@@ -1710,36 +1742,75 @@ static bool fast_path_ok(int block_size, int head_dim, int groups) {
   return block_size == FBS && (head_dim == 64 || head_dim == 128) && groups >= 1 && groups <= 16;
 }
 
-// Eight waves per workgroup (four for GQA groups above 8, to bound the LDS
-// accumulators); enough splits to put about 2048 waves (two per SIMD) on the
-// chip, but no more than one per 4*nw blocks of the row (a split costs a
-// partial publish, an arrival and a merge, three dependent memory round
-// trips, which only pays off when each split streams several tiles per
-// wave), and enough that no split's list exceeds MAX_LIST.
-static Plan plan_launch(int batch, int kv_heads, int num_blocks, int groups, int splits_hint) {
-  Plan pl;
-  pl.nw = groups <= 8 ? 8 : 4;
-  const int64_t units = std::max<int64_t>(1, int64_t(batch) * kv_heads);
-  int splits;
-  if (splits_hint > 0) {
-    splits = splits_hint;
-  } else {
-    const int64_t target_waves = 2048;
-    splits = int(std::max<int64_t>(1, (target_waves + units * pl.nw - 1) / (units * pl.nw)));
-    splits = std::min(splits, std::max(1, num_blocks / (4 * pl.nw)));
-    // Rows under 12 tiles per wave stay whole: at 64 blocks one workgroup
-    // per kv head took 6.96 us against 7.78 us for two splits (9.69 against
-    // 12.71 us with score sums, which a split launch finalises in a second
-    // launch); from 128 blocks on the splits above win.
-    if (num_blocks < 12 * pl.nw) splits = 1;
+// The fewest splits whose lists hold any row of num_blocks: a split's list
+// holds ceil(hot / splits) + ceil(warm / splits) entries, at most
+// ceil(num_blocks / splits) + 1; MAX_LIST - 1 blocks per split keep the HOT
+// (front) and WARM (back) halves of the list apart.
+static int min_splits(int num_blocks) { return std::max(1, (num_blocks + MAX_LIST - 2) / (MAX_LIST - 1)); }
+
+// Splits of a launch in the smallest workspace that is accepted: the hint, or
+// enough to put about 2048 waves on the chip with at least four tiles per
+// wave.  (A launch takes the plan below when its workspace has room.)
+static int required_splits(int64_t units, int num_blocks, int groups, int splits_hint) {
+  const int nw = groups <= 8 ? 8 : 4;
+  int64_t splits = splits_hint;
+  if (splits_hint <= 0) {
+    splits = std::max<int64_t>(1, (2048 + units * nw - 1) / (units * nw));
+    splits = std::min<int64_t>(splits, std::max(1, num_blocks / (4 * nw)));
+    if (num_blocks < 12 * nw) splits = 1;
   }
-  // A split's list holds ceil(hot / splits) + ceil(warm / splits) entries,
-  // at most ceil(num_blocks / splits) + 1: MAX_LIST - 1 blocks per split keep
-  // the HOT (front) and WARM (back) halves of the list apart.
-  splits = std::max(splits, (num_blocks + MAX_LIST - 2) / (MAX_LIST - 1));
-  splits = std::min(splits, std::max(1, num_blocks));
-  pl.splits = std::max(1, splits);
-  return pl;
+  splits = std::max<int64_t>(splits, min_splits(num_blocks));
+  return int(std::max<int64_t>(1, std::min<int64_t>(splits, num_blocks)));
+}
+
+// Expected time (us, less the launch itself) of a launch with nw waves per
+// workgroup and s splits per unit.  A CU moves about 26 B/ns whether one or
+// two workgroups and four or eight waves stream on it, so what counts is how
+// many workgroups the busiest CU gets, how many of them run together (by
+// registers: one of eight waves at head_dim 128, two at 64; twice as many of
+// four), and each pass's fixed part (list build, first loads, wave merge).
+// A split adds its publication, arrival and merge, and with score sums the
+// finalisation launch.  The constants are a fit to 6,192 timings (16
+// unit counts from 4 to 1024, ten row lengths from 9 to 2048 blocks, up to 12
+// split counts, both wave counts and head dims, with and without score sums;
+// 10 % HOT, 60 % WARM): over these shapes the plan chosen by it is on average
+// 1 % slower than the fastest measured one, where aiming at 2048 waves with
+// eight per workgroup was 15 % slower (head_dim 64: 9 %, with score sums 17 %;
+// up to 2.1x: 248 units made 496 workgroups of 256 that fit at a time).
+static double plan_cost(int64_t units, int num_blocks, int head_dim, bool scores, int nw, int s) {
+  const double per_block = head_dim == 64 ? 0.038 : 0.091;   // a block's tiles at a CU's rate
+  const double per_wave = 0.231;                             // a block's round trips in one wave
+  const double fixed = nw == 4 ? 6.0 : 6.4;
+  const int64_t room = (head_dim == 64 ? 2 : 1) * (nw == 4 ? 2 : 1);
+  const int64_t on_cu = (units * s + 255) / 256;
+  const int64_t passes = (on_cu + room - 1) / room;
+  const double refill = room == 1 ? 1.0 : nw == 4 ? 1.8 : 0.3;   // a further pass against the first
+  const double blocks = double(num_blocks) / s;
+  // One pass with so many workgroups together on the CU.  Four waves alone
+  // stream 3 % slower than eight (256 units of 1024 blocks: 145 against 141
+  // us), three workgroups of four where four fit (head_dim 64) 8 % (632
+  // units of 496 blocks: 88.8 against 81.8).
+  auto pass = [&](int64_t together) {
+    const double slower = nw == 4 && together == 1 && s == 1 ? 1.03 : nw == 4 && room == 4 && together == 3 ? 1.08 : 1.0;
+    return std::max(slower * per_block * blocks * together, per_wave * blocks / nw);
+  };
+  double t = fixed + (passes - 1) * (fixed * refill + pass(std::min(on_cu, room))) +
+             pass(on_cu - (passes - 1) * room);
+  if (s > 1)
+    t += 1.7 + (scores ? (nw == 4 ? 4.9 : 4.1) : 0.0) + 1.5 * ((s + MERGE_UNROLL - 1) / MERGE_UNROLL) +
+         0.3 * (std::min(on_cu, room) - 1);
+  // Rows longer than one pass of the list build (with score sums, the blanks
+  // of the later passes are written one by one).
+  t += ((num_blocks - 1) / (PRE_CHUNKS * nw * 64)) * (scores ? 3.5 : 1.0);
+  return t;
+}
+
+// Split counts a plan may take: at most MAX_PLAN_GRID workgroups, four blocks
+// per split.
+constexpr int PLAN_SPLITS[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32};
+constexpr int64_t MAX_PLAN_GRID = 1024;
+static bool plan_split_ok(int64_t units, int num_blocks, int s) {
+  return s == 1 || (units * s <= MAX_PLAN_GRID && s <= num_blocks / 4);
 }
 
 struct WsLayout {
@@ -1747,23 +1818,22 @@ struct WsLayout {
 };
 
 static WsLayout ws_layout(int batch, int num_heads, int kv_heads, int num_blocks, int block_size,
-                          int head_dim, bool scores, int splits_hint) {
+                          int head_dim, bool scores, int splits) {
   WsLayout l{};
   const int groups = num_heads / std::max(kv_heads, 1);
   auto up = [](int64_t x) { return (x + 255) & ~int64_t(255); };
   l.err = 0;
   int64_t off = 256;
   if (fast_path_ok(block_size, head_dim, groups)) {
-    const Plan pl = plan_launch(batch, kv_heads, num_blocks, groups, splits_hint);
     const int64_t units = int64_t(batch) * kv_heads;
     // The arrival counters come first and have the same place and size in
     // every layout, so a launch of any shape finds them zero.
     l.cnt = off;
     off = up(off + int64_t(MAX_SPLIT_UNITS) * 4);
     l.acc = off;
-    if (pl.splits > 1) off = up(off + units * pl.splits * groups * head_dim * 4);
+    if (splits > 1) off = up(off + units * splits * groups * head_dim * 4);
     l.ml = off;
-    if (pl.splits > 1) off = up(off + units * pl.splits * groups * 2 * 4);
+    if (splits > 1) off = up(off + units * splits * groups * 2 * 4);
     l.stage = off;
     if (scores) off = up(off + int64_t(batch) * num_heads * num_blocks * 2 * 4);
   } else {
@@ -1771,6 +1841,48 @@ static WsLayout ws_layout(int batch, int num_heads, int kv_heads, int num_blocks
   }
   l.total = off;
   return l;
+}
+
+// Wave and split counts of a fast-path launch: the cheapest by plan_cost whose
+// workspace fits workspace_bytes (that of required_splits always does); a
+// split hint fixes the splits.  GQA groups above 8 take four waves, to bound
+// the LDS accumulators.
+static Plan plan_launch(int batch, int num_heads, int kv_heads, int num_blocks, int block_size, int head_dim,
+                        bool scores, int splits_hint, int64_t workspace_bytes) {
+  const int groups = num_heads / kv_heads;
+  const int64_t units = int64_t(batch) * kv_heads;
+  Plan best{4, required_splits(units, num_blocks, groups, splits_hint)};
+  double best_cost = 1e300;
+  auto consider = [&](int s) {
+    for (int nw = 8; nw >= 4; nw -= 4) {
+      if (nw == 8 && groups > 8) continue;
+      const double c = plan_cost(units, num_blocks, head_dim, scores, nw, s);
+      if (c < best_cost) {
+        best_cost = c;
+        best = Plan{nw, s};
+      }
+    }
+  };
+  consider(best.splits);
+  if (splits_hint > 0) return best;
+  const int lo = min_splits(num_blocks);
+  for (int s : PLAN_SPLITS) {
+    if (s < lo || !plan_split_ok(units, num_blocks, s)) continue;
+    if (ws_layout(batch, num_heads, kv_heads, num_blocks, block_size, head_dim, scores, s).total > workspace_bytes)
+      break;
+    consider(s);
+  }
+  return best;
+}
+
+// Splits that the reported workspace has room for: whatever plan_launch may
+// take for this many blocks or fewer.
+static int reported_splits(int64_t units, int num_blocks, int groups, int splits_hint) {
+  int splits = required_splits(units, num_blocks, groups, splits_hint);
+  if (splits_hint <= 0)
+    for (int s : PLAN_SPLITS)
+      if (plan_split_ok(units, num_blocks, s)) splits = std::max(splits, s);
+  return splits;
 }
 
 template <int D, int WF, bool SC, bool CZ, typename QT, int NW>
@@ -1844,8 +1956,9 @@ extern "C" int64_t tierkv_decode_workspace_bytes(int32_t batch, int32_t num_head
                                                  int32_t with_scores, int32_t splits_hint) {
   if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_blocks <= 0 || block_size <= 0 || head_dim <= 0)
     return -1;
-  return ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, with_scores != 0,
-                   hint_splits(splits_hint)).total;
+  const int splits = reported_splits(int64_t(batch) * num_kv_heads, num_blocks, num_heads / num_kv_heads,
+                                     hint_splits(splits_hint));
+  return ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, with_scores != 0, splits).total;
 }
 
 // Every argument check of tierkv_decode_attention, before anything is
@@ -1886,9 +1999,10 @@ int32_t tierkv::decode_check_args(
   if (int64_t(batch) * num_kv_heads > (int64_t(1) << 24))
     return fail(TIERKV_ERR_UNSUPPORTED, "batch * kv_heads too large");
   const bool scores = score_sums != nullptr;
-  const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores, splits_hint);
-  if (workspace_bytes < wl.total) return fail(TIERKV_ERR_WORKSPACE, "workspace too small");
   const int groups = num_heads / num_kv_heads;
+  const int splits = required_splits(int64_t(batch) * num_kv_heads, num_blocks, groups, splits_hint);
+  const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores, splits);
+  if (workspace_bytes < wl.total) return fail(TIERKV_ERR_WORKSPACE, "workspace too small");
   if (fast_path_ok(block_size, head_dim, groups) && table_stride <= 0x7fffffff) {
     const bool aligned = aligned16(hot_k) && aligned16(hot_v) && aligned16(warm_k) && aligned16(warm_v) &&
                          aligned16(query);
@@ -1898,15 +2012,14 @@ int32_t tierkv::decode_check_args(
                           reinterpret_cast<uintptr_t>(v_scale) | reinterpret_cast<uintptr_t>(v_zero);
       if (m & 7u) return fail(TIERKV_ERR_INVALID, "reference-format scale/zero pools must be 8-byte aligned");
     }
-    const Plan pl = plan_launch(batch, num_kv_heads, num_blocks, groups, splits_hint);
-    if (pl.splits > 0x3fff || num_kv_heads > 0xffff)
+    if (splits > 0x3fff || num_kv_heads > 0xffff)
       return fail(TIERKV_ERR_UNSUPPORTED, "more than 65535 kv heads or 16383 splits");
     int64_t seqs_per_chunk = batch;
-    if (pl.splits > 1) {
+    if (splits > 1) {
       seqs_per_chunk = MAX_SPLIT_UNITS / num_kv_heads;
       if (seqs_per_chunk < 1) return fail(TIERKV_ERR_UNSUPPORTED, "too many kv heads for a split launch");
     }
-    if (std::min<int64_t>(seqs_per_chunk, batch) * num_kv_heads * pl.splits > 0x7fffffff)
+    if (std::min<int64_t>(seqs_per_chunk, batch) * num_kv_heads * splits > 0x7fffffff)
       return fail(TIERKV_ERR_UNSUPPORTED, "grid too large");
     if (scores && int64_t(batch) * num_heads > 0x7fffffff) return fail(TIERKV_ERR_UNSUPPORTED, "grid too large");
   }
@@ -1934,7 +2047,12 @@ extern "C" int32_t tierkv_decode_attention(
                                         num_kv_heads, block_size, head_dim, splits_hint, workspace, workspace_bytes);
   if (rc0 != TIERKV_OK) return rc0;
   const bool scores = score_sums != nullptr;
-  const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores, splits_hint);
+  const bool fast = fast_path_ok(block_size, head_dim, num_heads / num_kv_heads) && table_stride <= 0x7fffffff;
+  // (alignment and launch limits: decode_check_args)
+  const Plan pl = fast ? plan_launch(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores,
+                                     splits_hint, workspace_bytes)
+                       : Plan{1, 1};
+  const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores, pl.splits);
 
   DecodeParams p{};
   p.q = query;
@@ -1974,9 +2092,7 @@ extern "C" int32_t tierkv_decode_attention(
   const bool cz = cold_mode == TIERKV_COLD_ZERO_LOGIT;
   const bool bf16 = query_dtype == TIERKV_DTYPE_BF16;
 
-  if (fast_path_ok(block_size, head_dim, p.groups) && table_stride <= 0x7fffffff) {
-    // (alignment and launch limits: decode_check_args)
-    const Plan pl = plan_launch(batch, num_kv_heads, num_blocks, p.groups, splits_hint);
+  if (fast) {
     p.splits = pl.splits;
     p.split_magic = 0;
     // Unsplit score launches keep the per-block statistics in LDS (up to
@@ -2023,7 +2139,7 @@ extern "C" int32_t tierkv_decode_attention(
     // Block stages are finalised inside the decode launch; list and
     // workspace stages by one workgroup per (sequence, q head) row.
     if (rc != TIERKV_OK || !scores || p.lds_stage == STAGE_LDS_BLOCK) return rc;
-    const int parts = score_parts(p.groups, pl.nw);
+    const int parts = score_parts(p.groups);
     const int64_t rows = int64_t(batch) * num_heads;
     const size_t lds = num_blocks <= FIN_LDS_BLOCKS ? size_t(num_blocks) * sizeof(float2) : 0;
     const int32_t stride32 = int32_t(table_stride);
@@ -2115,8 +2231,14 @@ extern "C" int32_t tierkv_decode_attention_noalloc(
     float scaling, int32_t splits_hint, void* stream_) {
   clear_error();
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-  const int64_t need = tierkv_decode_workspace_bytes(batch, num_heads, num_kv_heads, num_blocks, block_size,
-                                                     head_dim, score_sums != nullptr, splits_hint);
+  // Invalid shapes are left to tierkv_decode_attention's checks.
+  int64_t need = 0;
+  if (batch > 0 && num_heads > 0 && num_kv_heads > 0 && num_blocks > 0 && block_size > 0 && head_dim > 0) {
+    const int splits = required_splits(int64_t(batch) * num_kv_heads, num_blocks, num_heads / num_kv_heads,
+                                       hint_splits(splits_hint));
+    need = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, score_sums != nullptr,
+                     splits).total;
+  }
   if (need > STATIC_SCRATCH_BYTES)
     return fail(TIERKV_ERR_WORKSPACE, "tierkv_decode_attention_noalloc: this launch needs " + std::to_string(need) +
                                           " bytes of scratch; the allocation-free entry point holds " +

@@ -527,3 +527,54 @@ def test_workspace_reuse_across_shapes(device):
                      (split, {"return_scores": True}), (small, {"return_scores": True}),
                      (split, {"splits": 3}), (big, {}), (split, {})):
         _check(case, "absmax_i8", device, seqs=[0, case.batch - 1], **kw)
+
+
+# -- wave and split plans -----------------------------------------------------
+
+@pytest.mark.parametrize("batch,kv,groups,dim,nb,lens,fmt", [
+    (1, 4, 4, 128, 9, False, "absmax_i8"),     # four waves, one tile each
+    (2, 8, 4, 128, 64, True, "ref_u8"),        # four waves, six splits: two output elements per merging thread
+    (1, 4, 3, 64, 400, True, "ref_u8"),        # eight waves, sixteen splits; 192 elements in a 512-thread merge
+    (2, 2, 8, 128, 150, False, "absmax_i8"),   # four waves, 1024 elements per unit
+    (31, 8, 1, 64, 20, True, "absmax_i8"),     # 248 units, unsplit; one head per unit
+    (40, 8, 2, 64, 33, True, "ref_u8"),        # more units than CUs
+    (1, 1, 16, 128, 300, True, "ref_u8"),      # sixteen heads: four waves, eight elements per merging thread
+    (1, 2, 5, 128, 1100, False, "absmax_i8"),  # rows past one list pass of four waves; an odd group
+])
+def test_plans_match_oracle(device, batch, kv, groups, dim, nb, lens, fmt):
+    """Shapes on both sides of the plan's wave and split choices, with and
+    without score sums (those the same bits as an eight-fold split's)."""
+    g = torch.Generator().manual_seed(nb)
+    lengths = torch.randint(0, 17, (batch, nb), generator=g) if lens else None
+    case = W.make_tiered_case(f"plan_u{batch * kv}_g{groups}_d{dim}_nb{nb}", batch, kv * groups, kv, dim, nb,
+                              max(1, nb // 8), nb // 2, seed=nb + groups, lengths=lengths)
+    seqs = list(range(min(batch, 3)))
+    _check(case, fmt, device, cold_mode="zero_logit", seqs=seqs)
+    _, sums = _check(case, fmt, device, cold_mode="zero_logit", return_scores=True, seqs=seqs)
+    _, split = _check(case, fmt, device, cold_mode="zero_logit", return_scores=True, seqs=seqs, splits=min(8, nb))
+    assert torch.equal(sums.view(torch.int32), split.view(torch.int32)), "score sums depend on the plan"
+
+
+def test_smallest_accepted_workspace(device):
+    """A launch takes the split count its workspace has room for: the counters
+    alone (no partials) are accepted for a short row and give an unsplit
+    launch; less is refused before anything is launched."""
+    from paged_tierkv_amd import _lib
+    from paged_tierkv_amd.tierkv_hip import PreparedDecode
+
+    case = W.make_tiered_case("ws_min", 2, 32, 8, 128, 64, 8, 40, seed=3)
+    args = to_gpu_inputs(case, oracle_warm(case, "absmax_i8"), device)
+    plan = PreparedDecode(**args, cold_mode="masked")
+    smallest = 256 + 65536 * 4
+    assert plan.workspace.nbytes > smallest
+    want = plan.launch()[0].clone()
+    ws = torch.zeros(smallest, dtype=torch.uint8, device=device)
+    call = lambda n: _lib.lib().tierkv_decode_attention(*plan._args[:-2], ws.data_ptr(), n, _lib.stream_of(device))
+    plan.out.zero_()
+    assert call(smallest) == _lib.TIERKV_OK
+    torch.cuda.synchronize()
+    assert_close(plan.out.float().cpu().numpy(), want.float().cpu().numpy(), what="unsplit launch")
+    plan.out.zero_()
+    assert call(smallest - 1) == _lib.TIERKV_ERR_WORKSPACE
+    torch.cuda.synchronize()
+    assert int(plan.out.count_nonzero()) == 0

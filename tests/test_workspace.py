@@ -94,3 +94,16 @@ def test_graph_runner_reserves_before_capture(monkeypatch):
     runner = hf_llama.DecodeGraphRunner(Model(), Rt())
     assert calls == [32]
     assert runner.rt.fixed_launch_bound
+
+
+@pytest.mark.parametrize("batch,heads,kv,dim", [(1, 32, 4, 64), (12, 32, 8, 128), (31, 32, 8, 128), (3, 16, 16, 64),
+                                                (2, 64, 4, 128), (200, 8, 8, 128)])
+@pytest.mark.parametrize("scores", [False, True])
+def test_reported_bytes_cover_every_shorter_row(batch, heads, kv, dim, scores):
+    """The split count a launch takes is not monotonic in its row length; the
+    reported workspace is, so one sized for the longest row fits every launch."""
+    last = 0
+    for nb in list(range(1, 140)) + [143, 144, 255, 256, 257, 400, 511, 512, 768, 1024, 1025, 2048, 2600, 5000]:
+        need = DecodeWorkspace.bytes_for(batch, heads, kv, nb, dim, return_scores=scores)
+        assert need >= last, (nb, need, last)
+        last = need
