@@ -172,6 +172,20 @@ TIERKV_API int32_t tierkv_demote_to_warm(
     int32_t* block_table, int32_t* block_states, const int32_t* table_pos,
     int32_t num_kv_heads, int32_t block_size, int32_t head_dim, void* stream);
 
+/* Quantization of a prompt's blocks straight into WARM slots, without fp16
+ * tiles in between: write_warm_block (tierkv_policy.py:969-1002) as
+ * append_prefill_with_policy (1722-1766) calls it, batched.  Job i quantizes
+ * tokens [src_tok[i], src_tok[i] + lengths[i]) of sequence src_seq[i] of the
+ * fp16 sources src_k/src_v [src_seqs, kv_heads, src_tokens, head_dim] into
+ * warm slot dst_slot[i], with the codecs and pad_tail of
+ * tierkv_demote_to_warm.  Jobs out of range are skipped. */
+TIERKV_API int32_t tierkv_quantize_tokens(
+    const void* src_k, const void* src_v, int64_t src_seqs, int32_t src_tokens,
+    const int32_t* src_seq, const int32_t* src_tok, const int32_t* dst_slot, const int32_t* lengths, int32_t n,
+    void* warm_k, void* warm_v, int64_t warm_slots,
+    void* k_scale, void* k_zero, void* v_scale, void* v_zero, int32_t warm_format, int32_t pad_tail,
+    int32_t num_kv_heads, int32_t block_size, int32_t head_dim, void* stream);
+
 /* Promotion WARM -> HOT.  Replaces promote_to_hot (tierkv_policy.py:1087-1115,
  * 375-402) with dequantize_int8_to_fp16 (39-44): job i dequantizes the first
  * lengths[i] tokens of warm slot src_slot[i] into hot slot dst_slot[i]

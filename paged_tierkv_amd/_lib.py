@@ -85,6 +85,13 @@ SIGNATURES = {
         c_int32, c_int32,
         _P, _P, _P,
         c_int32, c_int32, c_int32, _P]),
+    "tierkv_quantize_tokens": (c_int32, [
+        _P, _P, c_int64, c_int32,
+        _P, _P, _P, _P, c_int32,
+        _P, _P, c_int64,
+        _P, _P, _P, _P,
+        c_int32, c_int32,
+        c_int32, c_int32, c_int32, _P]),
     "tierkv_promote_to_hot": (c_int32, [
         _P, _P, c_int64,
         _P, _P, _P, _P,

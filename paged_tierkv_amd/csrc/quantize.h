@@ -10,6 +10,11 @@ struct QuantJobs {
   const __half* src[2];      // K, V source tiles [src_tiles, H_kv, bs, D]
   int64_t src_tiles;
   const int32_t* src_index;
+  // Set: the sources are sequences [src_tiles, H_kv, src_tokens, D] and job i
+  // quantizes tokens [src_tok[i], src_tok[i] + lengths[i]) of sequence
+  // src_index[i].
+  const int32_t* src_tok;
+  int32_t src_tokens;
   const int32_t* dst_slot;
   const int32_t* lengths;
   void* warm[2];

@@ -38,6 +38,21 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 
 
 
+// First row of job's source tile for head h of K (kv 0) or V (kv 1), or NULL
+// when the job's source is out of range.  Only its first len rows may be
+// read: a prompt's last block ends with the prompt.
+__device__ __forceinline__ const __half* tile_source(const QuantJobs& q, int64_t job, int kv, int h, int len) {
+  const int64_t si = q.src_index[job];
+  if (si < 0 || si >= q.src_tiles) return nullptr;
+  int64_t row = (si * q.kv_heads + h) * int64_t(q.bs);
+  if (q.src_tok) {
+    const int t = q.src_tok[job];
+    if (t < 0 || t > q.src_tokens - len) return nullptr;
+    row = (si * q.kv_heads + h) * int64_t(q.src_tokens) + t;
+  }
+  return (kv ? q.src[1] : q.src[0]) + row * q.D;
+}
+
 // ABSMAX_I8: one workgroup per (job, kv head, K|V) tile.
 __global__ __launch_bounds__(QT) void demote_absmax_kernel(QuantJobs q) {
   __shared__ float red[QT / 64];
@@ -45,13 +60,13 @@ __global__ __launch_bounds__(QT) void demote_absmax_kernel(QuantJobs q) {
   if (q.n_dev && job >= *q.n_dev) return;
   const int h = blockIdx.y;
   const int kv = blockIdx.z;
-  const int64_t si = q.src_index[job];
   const int64_t di = q.dst_slot[job];
-  if (si < 0 || si >= q.src_tiles || di < 0 || di >= q.warm_slots) return;
   const int len = min(max(q.lengths[job], 0), q.bs);
+  const __half* tile = tile_source(q, job, kv, h, len);
+  if (!tile || di < 0 || di >= q.warm_slots) return;
   const int64_t E = int64_t(q.bs) * q.D;
   const int64_t valid = int64_t(len) * q.D;
-  const __half* src = q.src[kv] + (si * q.kv_heads + h) * E;
+  const __half* src = tile;
   int8_t* dst = reinterpret_cast<int8_t*>(q.warm[kv]) + (di * q.kv_heads + h) * E;
 
   float amax = 0.f;
@@ -86,13 +101,13 @@ __global__ __launch_bounds__(QT) void demote_absmax_vec_kernel(QuantJobs q) {
   if (q.n_dev && job >= *q.n_dev) return;
   const int h = blockIdx.y;
   const int kv = blockIdx.z;
-  const int64_t si = q.src_index[job];
   const int64_t di = q.dst_slot[job];
-  if (si < 0 || si >= q.src_tiles || di < 0 || di >= q.warm_slots) return;
   const int len = min(max(q.lengths[job], 0), q.bs);
+  const __half* tile = tile_source(q, job, kv, h, len);
+  if (!tile || di < 0 || di >= q.warm_slots) return;
   const int64_t E = int64_t(q.bs) * q.D;
   const int64_t valid = int64_t(len) * q.D;
-  const uint4* src = reinterpret_cast<const uint4*>(q.src[kv] + (si * q.kv_heads + h) * E);
+  const uint4* src = reinterpret_cast<const uint4*>(tile);
   uint2* dst = reinterpret_cast<uint2*>(reinterpret_cast<int8_t*>(q.warm[kv]) + (di * q.kv_heads + h) * E);
   const int64_t nvec = E / 8;
 
@@ -104,8 +119,8 @@ __global__ __launch_bounds__(QT) void demote_absmax_vec_kernel(QuantJobs q) {
   for (int i = 0; i < MAXV; ++i) {
     const int64_t vi = threadIdx.x + int64_t(i) * QT;
     if (vi < nvec) {
-      x[i] = src[vi];
       if (vi * 8 < valid) {
+        x[i] = src[vi];
         const uint32_t w4[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -236,14 +251,14 @@ __global__ __launch_bounds__(QT) void demote_absmax_wave_kernel(QuantJobs q, int
   const int rem = static_cast<int>(tile - job * tiles_per_job);
   const int kv = rem / q.kv_heads;
   const int h = rem - kv * q.kv_heads;
-  const int64_t si = q.src_index[job];
   const int64_t di = q.dst_slot[job];
-  if (si < 0 || si >= q.src_tiles || di < 0 || di >= q.warm_slots) return;
   const int len = min(max(q.lengths[job], 0), q.bs);
+  const __half* rows = tile_source(q, job, kv, h, len);
+  if (!rows || di < 0 || di >= q.warm_slots) return;
   const int64_t E = int64_t(q.bs) * q.D;
   const int nvec = static_cast<int>(E / 8);
   const int valid_vec = len * q.D / 8;
-  const u32x4* src = reinterpret_cast<const u32x4*>(q.src[kv] + (si * q.kv_heads + h) * E);
+  const u32x4* src = reinterpret_cast<const u32x4*>(rows);
   u32x2* dst = reinterpret_cast<u32x2*>(reinterpret_cast<int8_t*>(q.warm[kv]) + (di * q.kv_heads + h) * E);
 
   // Every source byte is read once and every code written once: non-temporal
@@ -312,12 +327,11 @@ __global__ __launch_bounds__(QT) void demote_ref_kernel(QuantJobs q) {
   if (q.n_dev && job >= *q.n_dev) return;
   const int h = blockIdx.y;
   const int kv = blockIdx.z;
-  const int64_t si = q.src_index[job];
   const int64_t di = q.dst_slot[job];
-  if (si < 0 || si >= q.src_tiles || di < 0 || di >= q.warm_slots) return;
   const int len = min(max(q.lengths[job], 0), q.bs);
+  const __half* tile = tile_source(q, job, kv, h, len);
+  if (!tile || di < 0 || di >= q.warm_slots) return;
   const int D = q.D;
-  const int64_t tile_src = (si * q.kv_heads + h) * int64_t(q.bs);
   const int64_t tile_dst = (di * q.kv_heads + h) * int64_t(q.bs);
   uint8_t* codes = reinterpret_cast<uint8_t*>(q.warm[kv]);
   __half* scale = reinterpret_cast<__half*>(q.scale[kv]);
@@ -327,7 +341,7 @@ __global__ __launch_bounds__(QT) void demote_ref_kernel(QuantJobs q) {
   for (int r0 = 0; r0 < q.bs; r0 += rows_per_pass) {
     const int r = r0 + (threadIdx.x >> 4);
     const bool row_ok = r < q.bs;
-    const __half* x = q.src[kv] + (tile_src + r) * D;
+    const __half* x = tile + int64_t(r) * D;
     float mn = INFINITY, mx = -INFINITY;
     if (row_ok && r < len) {
       for (int d = sub; d < D; d += 16) {
@@ -461,15 +475,15 @@ __global__ __launch_bounds__(QT) void demote_ref_wave_kernel(QuantJobs q, int32_
   const int rem = static_cast<int>(tile - job * tiles_per_job);
   const int kv = rem / q.kv_heads;
   const int h = rem - kv * q.kv_heads;
-  const int64_t si = q.src_index[job];
   const int64_t di = q.dst_slot[job];
-  if (si < 0 || si >= q.src_tiles || di < 0 || di >= q.warm_slots) return;
   const int len = min(max(q.lengths[job], 0), q.bs);
+  const __half* rows = tile_source(q, job, kv, h, len);
+  if (!rows || di < 0 || di >= q.warm_slots) return;
   const int R = 1 << r_log2;
   const int64_t E = int64_t(q.bs) * q.D;
   const int nvec = q.bs * R;
   const int valid_vec = len * R;
-  const u32x4* src = reinterpret_cast<const u32x4*>(q.src[kv] + (si * q.kv_heads + h) * E);
+  const u32x4* src = reinterpret_cast<const u32x4*>(rows);
   u32x2* dst = reinterpret_cast<u32x2*>(reinterpret_cast<uint8_t*>(q.warm[kv]) + (di * q.kv_heads + h) * E);
   __half* scale = reinterpret_cast<__half*>(q.scale[kv]) + (di * q.kv_heads + h) * int64_t(q.bs);
   __half* zero = reinterpret_cast<__half*>(q.zero[kv]) + (di * q.kv_heads + h) * int64_t(q.bs);
@@ -820,6 +834,45 @@ extern "C" int32_t tierkv_demote_to_warm(
   if (warm_format == TIERKV_WARM_REF_U8 && (!k_zero || !v_zero))
     return fail(TIERKV_ERR_INVALID, "reference format needs zero-point pools");
   return launch_demote(q, n, warm_format, stream);
+}
+
+extern "C" int32_t tierkv_quantize_tokens(
+    const void* src_k, const void* src_v, int64_t src_seqs, int32_t src_tokens,
+    const int32_t* src_seq, const int32_t* src_tok, const int32_t* dst_slot, const int32_t* lengths, int32_t n,
+    void* warm_k, void* warm_v, int64_t warm_slots,
+    void* k_scale, void* k_zero, void* v_scale, void* v_zero, int32_t warm_format, int32_t pad_tail,
+    int32_t num_kv_heads, int32_t block_size, int32_t head_dim, void* stream_) {
+  clear_error();
+  if (n < 0) return fail(TIERKV_ERR_INVALID, "negative job count");
+  if (n == 0) return TIERKV_OK;
+  if (!src_k || !src_v || !src_seq || !src_tok || !dst_slot || !lengths || !warm_k || !warm_v || !k_scale || !v_scale)
+    return fail(TIERKV_ERR_INVALID, "null pointer");
+  if (num_kv_heads <= 0 || block_size <= 0 || block_size > 64 || head_dim <= 0 || head_dim > 256 || src_tokens <= 0)
+    return fail(TIERKV_ERR_UNSUPPORTED, "block_size must be in [1, 64] and head_dim in [1, 256]");
+  if (n > 65535 * 64) return fail(TIERKV_ERR_UNSUPPORTED, "too many quantize jobs in one call");
+  if (warm_format == TIERKV_WARM_REF_U8 && (!k_zero || !v_zero))
+    return fail(TIERKV_ERR_INVALID, "reference format needs zero-point pools");
+  QuantJobs q{};
+  q.src[0] = reinterpret_cast<const __half*>(src_k);
+  q.src[1] = reinterpret_cast<const __half*>(src_v);
+  q.src_tiles = src_seqs;
+  q.src_index = src_seq;
+  q.src_tok = src_tok;
+  q.src_tokens = src_tokens;
+  q.dst_slot = dst_slot;
+  q.lengths = lengths;
+  q.warm[0] = warm_k;
+  q.warm[1] = warm_v;
+  q.warm_slots = warm_slots;
+  q.scale[0] = k_scale;
+  q.scale[1] = v_scale;
+  q.zero[0] = k_zero;
+  q.zero[1] = v_zero;
+  q.kv_heads = num_kv_heads;
+  q.bs = block_size;
+  q.D = head_dim;
+  q.pad_tail = pad_tail;
+  return launch_demote(q, n, warm_format, reinterpret_cast<hipStream_t>(stream_));
 }
 
 extern "C" int32_t tierkv_promote_to_hot(

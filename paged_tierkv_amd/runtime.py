@@ -30,6 +30,7 @@ import os
 
 from dataclasses import dataclass
 
+import numpy as np
 import torch
 
 from . import _lib, kernels
@@ -86,6 +87,25 @@ def recency_scores(num_blocks: int) -> list[float]:
     return s
 
 
+def _prefill_tiers(scores: np.ndarray, hot_budget: int, warm_budget: int, policy_mode: str) -> np.ndarray:
+    """``prefill_states`` of every row of scores [rows, n] at once (int32)."""
+    rows, n = scores.shape
+    out = np.full((rows, n), HOT_STATE, dtype=np.int32)
+    if n <= 2:
+        return out
+    if np.isnan(scores).any():   # no order among candidates: Python's sort decides
+        return np.array([prefill_states(n, r, hot_budget, warm_budget, policy_mode) for r in scores], dtype=np.int32)
+    order = np.argsort(-scores[:, 1:-1], axis=1, kind="stable")
+    rank = np.empty_like(order)
+    np.put_along_axis(rank, order, np.arange(n - 2)[None], axis=1)
+    extra = max(int(hot_budget) - 2, 0)
+    rest = WARM_STATE
+    if policy_mode == "hot_warm_cold":
+        rest = np.where(rank < extra + max(int(warm_budget), 0), WARM_STATE, COLD_STATE)
+    out[:, 1:-1] = np.where(rank < extra, HOT_STATE, rest)
+    return out
+
+
 def _strided_f16(t: torch.Tensor) -> torch.Tensor:
     """fp16 tensor whose head dimension is contiguous, with strides that are
     multiples of 8 elements and a 16-byte aligned start (copied otherwise)."""
@@ -114,6 +134,7 @@ class LayerStorage:
     hot_free: torch.Tensor    # [hot capacity] free-slot stack
     warm_free: torch.Tensor   # [warm capacity]
     ctl: torch.Tensor         # [4] hot_top, warm_top, error bits, last append applied
+    meta: torch.Tensor        # the int32 buffer the eight tensors above are views of
 
 
 class BatchedTieredKVRuntime:
@@ -185,6 +206,15 @@ class BatchedTieredKVRuntime:
             self.warm_per_seq = min(n, budget_blocks(self.warm_fraction, n) + hot_max + 2)
         self.hot_slots = self.batch * self.hot_per_seq
         self.warm_slots = max(1, self.batch * self.warm_per_seq)
+        # Where a layer's int32 tensors lie in its buffer (each 256-byte aligned).
+        self._meta_views, at = {}, 0
+        for name, shape in (("table", (self.batch, n)), ("states", (self.batch, n)), ("lengths", (self.batch, n)),
+                            ("nblocks", (self.batch,)), ("open", (self.batch,)), ("hot_free", (self.hot_slots,)),
+                            ("warm_free", (self.warm_slots,)), ("ctl", (4,))):
+            size = int(np.prod(shape))
+            self._meta_views[name] = (at, size, shape)
+            at += _ceil_div(size, 64) * 64
+        self._meta_len = at
         self.layers = [self._new_layer() for _ in range(self.num_layers)]
         # Host copy of the (lockstep) block count and open-block fill per layer,
         # so launch sizes and budgets need no device read-back.
@@ -231,19 +261,17 @@ class BatchedTieredKVRuntime:
             vs = torch.ones((self.warm_slots, kv, bs, 1), dtype=torch.float16, device=dev)
             kz = torch.zeros((self.warm_slots, kv, bs, 1), dtype=torch.float16, device=dev)
             vz = torch.zeros((self.warm_slots, kv, bs, 1), dtype=torch.float16, device=dev)
-        tab = (self.batch, self.max_blocks)
+        # The tables, counts, free stacks and control words are views of one
+        # buffer, so that a prefill replaces them with one copy.
+        meta = torch.zeros(self._meta_len, dtype=torch.int32, device=dev)
+        views = {name: meta[at: at + size].view(shape) for name, (at, size, shape) in self._meta_views.items()}
+        views["table"].fill_(-1)
+        views["states"].fill_(COLD_STATE)
         return LayerStorage(
             hot_k=torch.zeros(hot, dtype=torch.float16, device=dev),
             hot_v=torch.zeros(hot, dtype=torch.float16, device=dev),
             warm_k=wk, warm_v=wv, k_scale=ks, k_zero=kz, v_scale=vs, v_zero=vz,
-            table=torch.full(tab, -1, dtype=torch.int32, device=dev),
-            states=torch.full(tab, COLD_STATE, dtype=torch.int32, device=dev),
-            lengths=torch.zeros(tab, dtype=torch.int32, device=dev),
-            nblocks=torch.zeros(self.batch, dtype=torch.int32, device=dev),
-            open=torch.zeros(self.batch, dtype=torch.int32, device=dev),
-            hot_free=torch.zeros(self.hot_slots, dtype=torch.int32, device=dev),
-            warm_free=torch.zeros(self.warm_slots, dtype=torch.int32, device=dev),
-            ctl=torch.zeros(4, dtype=torch.int32, device=dev))
+            meta=meta, **views)
 
     def budgets(self, num_blocks: int) -> tuple[int, int]:
         hot = max(2, budget_blocks(self.hot_fraction, num_blocks))
@@ -270,73 +298,73 @@ class BatchedTieredKVRuntime:
         v = value_states.to(torch.float16).contiguous()
         hot_b, warm_b = self.budgets(n)
         if block_scores is None:
-            per_seq = [recency_scores(n)] * B
+            scores = np.array(recency_scores(n), dtype=np.float64)
         else:
-            sc = torch.as_tensor(block_scores, dtype=torch.float32).cpu()
-            per_seq = [sc.tolist()] * B if sc.ndim == 1 else [sc[b].tolist() for b in range(B)]
+            scores = torch.as_tensor(block_scores, dtype=torch.float32).cpu().numpy().astype(np.float64)
+        if scores.ndim == 1:
+            scores = scores[None]
+        elif scores.shape[0] < B:
+            raise IndexError("block_scores needs one row per sequence.")
+        if n > 2 and scores.shape[1] < n - 1:
+            raise IndexError("block_scores needs one score per candidate block.")
+        scores = np.pad(scores, ((0, 0), (0, max(n - scores.shape[1], 0))))   # the last block is no candidate
+        tiers = np.broadcast_to(_prefill_tiers(scores[:B, :n], hot_b, warm_b, self.policy_mode), (B, n))
         bs = self.block_size
-        table = torch.full((B, self.max_blocks), -1, dtype=torch.int32)
-        states = torch.full((B, self.max_blocks), COLD_STATE, dtype=torch.int32)
-        lengths = torch.zeros((B, self.max_blocks), dtype=torch.int32)
-        hot_jobs, warm_jobs = [], []
-        next_hot = next_warm = 0
-        for b in range(B):
-            tiers = prefill_states(n, per_seq[b], hot_b, warm_b, self.policy_mode)
-            for i, s in enumerate(tiers):
-                ln = min(bs, T - i * bs)
-                lengths[b, i] = ln
-                states[b, i] = s
-                if s == HOT_STATE:
-                    table[b, i] = next_hot
-                    hot_jobs.append((b, i * bs, ln, next_hot))
-                    next_hot += 1
-                elif s == WARM_STATE:
-                    table[b, i] = next_warm
-                    warm_jobs.append((b, i * bs, ln, next_warm))
-                    next_warm += 1
-        if next_hot > self.hot_slots or next_warm > self.warm_slots:
+        first = np.arange(n, dtype=np.int32) * bs               # each block's first token
+        count = np.minimum(T - first, bs).astype(np.int32)
+        # Slots in (sequence, block) order, per tier.
+        hot_at, warm_at = np.nonzero(tiers == HOT_STATE), np.nonzero(tiers == WARM_STATE)
+        nh, nw = len(hot_at[0]), len(warm_at[0])
+        if nh > self.hot_slots or nw > self.warm_slots:
             raise RuntimeError("prefill needs more slots than the runtime's pools hold.")
-        dev = self.device
-        if hot_jobs:
-            self._write_hot(k, v, hot_jobs, st.hot_k, st.hot_v)
-        if warm_jobs:
-            # WARM blocks: fp16 tiles staged once, quantized into their slots.
-            stage_k = torch.zeros((len(warm_jobs), kv, bs, d), dtype=torch.float16, device=dev)
-            stage_v = torch.zeros_like(stage_k)
-            self._write_hot(k, v, [(b, t0, ln, j) for j, (b, t0, ln, _) in enumerate(warm_jobs)], stage_k, stage_v)
-            kernels.demote_to_warm(stage_k, stage_v, list(range(len(warm_jobs))), [w[3] for w in warm_jobs],
-                                   [w[2] for w in warm_jobs], st.warm_k, st.warm_v, st.k_scale, st.k_zero,
-                                   st.v_scale, st.v_zero, warm_format=self.warm_format, pad_tail=True)
-        st.table.copy_(table)
-        st.states.copy_(states)
-        st.lengths.copy_(lengths)
-        st.nblocks.fill_(n)
-        st.open.zero_()      # decode tokens start a new block (tierkv_policy.py:1764-1766)
+        # One host buffer for everything the device needs: the layer's int32
+        # tensors as they lie in its buffer, then the copy jobs' columns
+        # (sequence, first token, count, slot, position) and the quantize jobs'
+        # (sequence, first token, count, slot).  It is pinned and copied once;
+        # building the tables entry by entry and uploading every list by itself
+        # took 9 ms of host time per layer (16 sequences of 128 blocks).
+        m = self._meta_len
+        host = torch.empty(m + 5 * nh + 4 * nw, dtype=torch.int32, pin_memory=True)
+        buf = host.numpy()
+        buf[:m] = 0
+        part = {name: buf[at: at + size].reshape(shape) for name, (at, size, shape) in self._meta_views.items()}
+        part["table"][:] = -1
+        part["states"][:] = COLD_STATE
+        part["states"][:, :n] = tiers
+        part["lengths"][:, :n] = count
+        part["table"][hot_at] = np.arange(nh)
+        part["table"][warm_at] = np.arange(nw)
+        part["nblocks"][:] = n
+        # (open stays 0: decode tokens start a new block, tierkv_policy.py:1764-1766)
+        # Free stacks: popping from the top yields the lowest free slot first.
+        part["hot_free"][: self.hot_slots - nh] = np.arange(self.hot_slots - 1, nh - 1, -1)
+        part["warm_free"][: self.warm_slots - nw] = np.arange(self.warm_slots - 1, nw - 1, -1)
+        part["ctl"][:] = (self.hot_slots - nh, self.warm_slots - nw, 0, 0)
+        hot_jobs = buf[m: m + 5 * nh].reshape(5, nh)
+        hot_jobs[:] = hot_at[0], first[hot_at[1]], count[hot_at[1]], np.arange(nh), np.zeros(nh)
+        warm_jobs = buf[m + 5 * nh:].reshape(4, nw)
+        warm_jobs[:] = warm_at[0], first[warm_at[1]], count[warm_at[1]], np.arange(nw)
+        dev = host.to(self.device, non_blocking=True)
+        lib, stream = _lib.lib(), _lib.stream_of(self.device)
+        if nh:
+            seq, tok, cnt, slot, pos = (_lib.ptr(r) for r in dev[m: m + 5 * nh].view(5, nh))
+            rc = lib.tierkv_write_hot_tokens(_lib.ptr(k), _lib.ptr(v), B, T, seq, tok, cnt, slot, pos, nh, 1,
+                                             _lib.ptr(st.hot_k), _lib.ptr(st.hot_v), self.hot_slots, kv, bs, d, stream)
+            _lib.check(rc, "tierkv_write_hot_tokens")
+        if nw:
+            # WARM blocks are quantized straight from the prompt.
+            seq, tok, cnt, slot = (_lib.ptr(r) for r in dev[m + 5 * nh:].view(4, nw))
+            rc = lib.tierkv_quantize_tokens(_lib.ptr(k), _lib.ptr(v), B, T, seq, tok, slot, cnt, nw,
+                                            _lib.ptr(st.warm_k), _lib.ptr(st.warm_v), self.warm_slots,
+                                            _lib.ptr(st.k_scale), _lib.ptr(st.k_zero), _lib.ptr(st.v_scale),
+                                            _lib.ptr(st.v_zero), kernels.WARM_FORMATS[self.warm_format], 1,
+                                            kv, bs, d, stream)
+            _lib.check(rc, "tierkv_quantize_tokens")
+        st.meta.copy_(dev[:m])
         self._blocks[layer] = n
         self._open_tokens[layer] = 0
-        # Free stacks: popping from the top yields the lowest free slot first.
-        st.hot_free[: self.hot_slots - next_hot].copy_(
-            torch.arange(self.hot_slots - 1, next_hot - 1, -1, dtype=torch.int32))
-        st.warm_free[: self.warm_slots - next_warm].copy_(
-            torch.arange(self.warm_slots - 1, next_warm - 1, -1, dtype=torch.int32))
-        st.ctl.copy_(torch.tensor([self.hot_slots - next_hot, self.warm_slots - next_warm, 0, 0],
-                                  dtype=torch.int32))
         if layer == self.num_layers - 1:
             self.seq_len = T
-
-    def _write_hot(self, k, v, jobs, dst_k, dst_v) -> None:
-        lib = _lib.lib()
-        cols = list(zip(*jobs))
-        dev = self.device
-        arr = [torch.tensor(c, dtype=torch.int32, device=dev) for c in cols]
-        src_seq, src_tok, count, slot = arr
-        zeros = torch.zeros_like(slot)
-        rc = lib.tierkv_write_hot_tokens(
-            _lib.ptr(k), _lib.ptr(v), int(k.shape[0]), int(k.shape[2]),
-            _lib.ptr(src_seq), _lib.ptr(src_tok), _lib.ptr(count), _lib.ptr(slot), _lib.ptr(zeros),
-            len(jobs), 1, _lib.ptr(dst_k), _lib.ptr(dst_v), int(dst_k.shape[0]),
-            self.kv_heads, self.block_size, self.head_dim, _lib.stream_of(dev))
-        _lib.check(rc, "tierkv_write_hot_tokens")
 
     # -- decode -------------------------------------------------------------
 
