@@ -164,7 +164,10 @@ def tier_labels(scores: torch.Tensor, cur_states: torch.Tensor, hot_budget: int,
     cur = (cur_states.unsqueeze(0) if cur_states.ndim == 1 else cur_states).to(torch.int32).contiguous()
     batch, n = (int(x) for x in sc.shape)
     if out is None:
-        out = cur.clone()
+        # The kernel writes every entry below n: only a wider or taller table
+        # needs its other entries copied first (a device copy, about 5 us of a
+        # 17 us scoring call).
+        out = torch.empty_like(cur) if tuple(cur.shape) == (batch, n) else cur.clone()
     else:
         out = out.unsqueeze(0) if out.ndim == 1 else out
     rc = lib.tierkv_tier_labels(_lib.ptr(sc), _lib.ptr(cur), _lib.ptr(out), int(cur.shape[-1]), batch, n,

@@ -129,3 +129,18 @@ def test_scores_from_sums_bit_exact(device):
     assert np.array_equal(_bits(got), _bits(exp))
     one = kernels.block_scores_from_sums(sums[0].to(device), lens[0].to(device), 10).cpu().numpy()
     assert np.array_equal(_bits(one), _bits(exp[0, :10]))
+
+
+@pytest.mark.parametrize("rows,width", [(2, 9), (2, 12), (3, 9)])
+def test_labels_keep_entries_outside_the_ranked_blocks(device, rows, width):
+    """Entries past n, and rows past the scores', come back unchanged; a table
+    of exactly the scores' shape is written whole."""
+    batch, n = 2, 9
+    g = torch.Generator().manual_seed(rows * width)
+    scores = torch.rand((batch, n), generator=g)
+    cur = torch.randint(0, 3, (rows, width), generator=g, dtype=torch.int32)
+    got = kernels.tier_labels(scores.to(device), cur.to(device), 4, 3).cpu()
+    want = cur.clone()
+    want[:batch, :n] = torch.from_numpy(opolicy.tier_labels(scores.numpy(), cur[:batch, :n].numpy(), 4, 3,
+                                                            "hot_warm_cold"))
+    assert torch.equal(got, want)
