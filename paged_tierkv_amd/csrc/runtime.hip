@@ -255,7 +255,21 @@ __device__ __forceinline__ uint4 kv_finish(const AppendParams& a, const KVItem& 
   return r.x;
 }
 
-constexpr int APPEND_NIT = APPEND_MAX_BATCH / RT;     // sequences per thread, at most
+// Threads of the append's bookkeeping: one wave for up to 64 sequences (its
+// scan needs no barrier), else RT threads.
+constexpr int APPEND_WAVE = 64;
+
+// block_scan for a workgroup of NT threads.
+template <int NT>
+__device__ __forceinline__ int append_scan(int v, int* sh, int* total) {
+  if constexpr (NT == APPEND_WAVE) {
+    const int x = wave_inclusive_scan(v);
+    *total = __builtin_amdgcn_readlane(x, 63);
+    return x;
+  } else {
+    return block_scan(v, sh, total);
+  }
+}
 
 // Append bookkeeping (one workgroup): per sequence, the open block (flagged,
 // last, HOT, not full) is filled first, then new HOT blocks popped from the
@@ -270,19 +284,21 @@ constexpr int APPEND_NIT = APPEND_MAX_BATCH / RT;     // sequences per thread, a
 // caller expects every sequence to hold (0: none).  With it, the entries of
 // the sequences' last blocks are loaded together with their counts, and
 // only a sequence whose count differs takes another round trip.
-__global__ __launch_bounds__(RT) void append_plan_kernel(const int32_t* r_nblocks, const int32_t* r_open,
+template <int NT>
+__global__ __launch_bounds__(NT) void append_plan_kernel(const int32_t* r_nblocks, const int32_t* r_open,
                                                          const int32_t* r_lengths, const int32_t* r_states,
                                                          const int32_t* r_table, int32_t stride32, int32_t hint,
                                                          int32_t batch, AppendParams a) {
+  constexpr int NIT = NT == APPEND_WAVE ? 1 : APPEND_MAX_BATCH / NT;   // sequences per thread, at most
   __shared__ int sh[RT / 64 + 1];
   __shared__ int s_ok;
   const int tid = threadIdx.x;
-  const int nit = (batch + RT - 1) / RT;
-  int nb[APPEND_NIT], opn[APPEND_NIT], ln[APPEND_NIT], stt[APPEND_NIT], slot_open[APPEND_NIT];
+  const int nit = (batch + NT - 1) / NT;
+  int nb[NIT], opn[NIT], ln[NIT], stt[NIT], slot_open[NIT];
 #pragma unroll
-  for (int it = 0; it < APPEND_NIT; ++it) {
+  for (int it = 0; it < NIT; ++it) {
     if (it < nit) {
-      const int b = min(it * RT + tid, batch - 1);
+      const int b = min(it * NT + tid, batch - 1);
       const int64_t o = int64_t(b) * stride32 + min(max(hint - 1, 0), stride32 - 1);
       nb[it] = r_nblocks[b];
       opn[it] = r_open[b];
@@ -295,12 +311,12 @@ __global__ __launch_bounds__(RT) void append_plan_kernel(const int32_t* r_nblock
   const int B = batch, bs = a.bs, T = a.T;
   const int top = a.ctl[0];
   if (tid == 0) s_ok = 1;
-  int room[APPEND_NIT], len_open[APPEND_NIT], need[APPEND_NIT], excl[APPEND_NIT];
+  int room[NIT], len_open[NIT], need[NIT], excl[NIT];
   // Sequences whose count is not the hint reload their last block's entries.
 #pragma unroll
-  for (int it = 0; it < APPEND_NIT; ++it) {
+  for (int it = 0; it < NIT; ++it) {
     if (it < nit && nb[it] != hint) {
-      const int b = min(it * RT + tid, B - 1);
+      const int b = min(it * NT + tid, B - 1);
       const int64_t o = int64_t(b) * stride32 + min(max(nb[it] - 1, 0), stride32 - 1);
       ln[it] = r_lengths[o];
       stt[it] = r_states[o];
@@ -308,9 +324,9 @@ __global__ __launch_bounds__(RT) void append_plan_kernel(const int32_t* r_nblock
     }
   }
 #pragma unroll
-  for (int it = 0; it < APPEND_NIT; ++it) {
+  for (int it = 0; it < NIT; ++it) {
     room[it] = len_open[it] = need[it] = excl[it] = 0;
-    const int b = it * RT + tid;
+    const int b = it * NT + tid;
     if (it < nit && b < B) {
       if (nb[it] > 0 && nb[it] <= stride32 && opn[it] != 0) {
         const int len = min(max(ln[it], 0), bs);
@@ -327,12 +343,12 @@ __global__ __launch_bounds__(RT) void append_plan_kernel(const int32_t* r_nblock
   __syncthreads();
   int run = 0;
 #pragma unroll
-  for (int it = 0; it < APPEND_NIT; ++it) {
+  for (int it = 0; it < NIT; ++it) {
     if (it < nit) {
-      const int b = it * RT + tid;
+      const int b = it * NT + tid;
       if (b < B && (nb[it] < 0 || nb[it] + need[it] > stride32)) s_ok = 0;
       int tot;
-      excl[it] = run + block_scan(need[it], sh, &tot) - need[it];
+      excl[it] = run + append_scan<NT>(need[it], sh, &tot) - need[it];
       run += tot;
     }
   }
@@ -346,8 +362,8 @@ __global__ __launch_bounds__(RT) void append_plan_kernel(const int32_t* r_nblock
   }
   // Table entries; new blocks pop the stack in sequence order.
 #pragma unroll
-  for (int it = 0; it < APPEND_NIT; ++it) {
-    const int b = it * RT + tid;
+  for (int it = 0; it < NIT; ++it) {
+    const int b = it * NT + tid;
     if (it < nit && b < B) {
       const int take_open = min(room[it], T);
       if (take_open > 0) a.lengths[int64_t(b) * a.stride + nb[it] - 1] = len_open[it] + take_open;
@@ -411,15 +427,22 @@ __global__ __launch_bounds__(CT) void append_copy_kernel(AppendParams a, int32_t
   __builtin_amdgcn_sched_barrier(0);
   if (!applied || blk < 0) return;
   // Walk back over the row list to the token's block.
+  // (a block's length and slot are read together: one round trip when the
+  // token lies in the last block, as a decode step's does).
   int r = T - 1 - it.t;
-  int len = min(max(a.lengths[int64_t(it.b) * a.stride + blk], 0), bs);
+  const int64_t row = int64_t(it.b) * a.stride;
+  int len = a.lengths[row + blk], slot32 = a.table[row + blk];
+  __builtin_amdgcn_sched_barrier(0);
+  len = min(max(len, 0), bs);
   while (r >= len && blk > 0) {
     r -= len;
     --blk;
-    len = min(max(a.lengths[int64_t(it.b) * a.stride + blk], 0), bs);
+    len = a.lengths[row + blk];
+    slot32 = a.table[row + blk];
+    len = min(max(len, 0), bs);
   }
   if (r >= len) return;
-  const int64_t slot = a.table[int64_t(it.b) * a.stride + blk];
+  const int64_t slot = slot32;
   if (slot < 0 || slot >= a.hot_slots) return;
   __half* pool = it.kv ? a.hot[1] : a.hot[0];
   reinterpret_cast<uint4*>(pool + ((slot * H + it.h) * int64_t(bs) + (len - 1 - r)) * D)[it.c] =
@@ -913,8 +936,12 @@ template <bool ROPE>
 static int32_t launch_append(const AppendParams& a, const int32_t* nblocks, const int32_t* open,
                              const int32_t* lengths, const int32_t* states, const int32_t* table, int32_t stride32,
                              int32_t hint, int32_t batch, int q_groups, hipStream_t stream) {
-  hipLaunchKernelGGL(append_plan_kernel, dim3(1), dim3(RT), 0, stream, nblocks, open, lengths, states, table, stride32,
-                     hint, batch, a);
+  if (batch <= APPEND_WAVE)
+    hipLaunchKernelGGL(append_plan_kernel<APPEND_WAVE>, dim3(1), dim3(APPEND_WAVE), 0, stream, nblocks, open, lengths,
+                       states, table, stride32, hint, batch, a);
+  else
+    hipLaunchKernelGGL(append_plan_kernel<RT>, dim3(1), dim3(RT), 0, stream, nblocks, open, lengths, states, table,
+                       stride32, hint, batch, a);
   const int32_t rc = check_launch("append_plan_kernel");
   if (rc != TIERKV_OK) return rc;
   const int64_t total_kv = int64_t(batch) * 2 * a.kv_heads * a.T * (a.D / 8);
