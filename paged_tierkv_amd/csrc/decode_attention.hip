@@ -808,8 +808,8 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
     }
   };
   if (tid == 0) {
-    s_next[0] = 0;
-    s_next[1] = 0;
+    s_next[0] = TIERKV_NBW * nw;   // the first positions are fixed (tile loops)
+    s_next[1] = TIERKV_NBH * nw;
     for (int i = 0; i < MAX_WAVES; ++i) s_prog[i] = 0;
   }
 
@@ -1120,8 +1120,16 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
   // The tile loops are instantiated once per hand-out (one uniform branch
   // here): a check of the mode inside the loops cost the default hand-out
   // 0.7 us at C3.
+  const int wu = uniform(w);
   auto tile_loops = [&](auto DET) {
-    int kc0 = 0, kc1 = 0;
+    // The first NBW (NBH) positions of a wave are fixed in both modes (the
+    // counters start past them).  The wave index is a scalar here: a position
+    // computed per lane makes its tile's buffer size, 0 for a dead step, a
+    // per-lane value and every load a loop over the lanes' resources
+    // (deterministic launches, 128 units of 144 blocks in two splits: 19.5 ->
+    // 18.4 us; 4 units of 9 blocks 7.3 -> 6.2).
+    auto fixed_pos = [&](int c, int k) -> int { return (c ? nw - 1 - wu : wu) + nw * k; };
+    int kc0 = TIERKV_NBW, kc1 = TIERKV_NBH;
     auto grab = [&](int c) -> int {
       if constexpr (decltype(DET)::value) {
         const int k = c ? kc1++ : kc0++;
@@ -1130,7 +1138,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
           if (uniform(s_prog[w ^ 4]) > kc0 + kc1) __builtin_amdgcn_s_setprio(1);
           else __builtin_amdgcn_s_setprio(0);
         }
-        return (c ? nw - 1 - w : w) + nw * k;
+        return fixed_pos(c, k);
       } else {
         int v = 0;
         if (lane == 0) v = atomicAdd(&s_next[c], 1);
@@ -1145,7 +1153,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
     int4 hne = make_int4(0, 0, 0, 0);   // next HOT entry to load and whether it is live
     bool hnl = false;
     if (nhot > 0) {
-      int gi = grab(1);
+      int gi = fixed_pos(1, 0);
       hne = s_list[min(gi, nhot - 1)];
       hnl = gi < nhot;
 #pragma unroll
@@ -1154,7 +1162,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
         lh[k] = hnl;
         load_hot<D>(p, kvh, uniform(hne.y), lane, th[k], hnl);
         __builtin_amdgcn_sched_barrier(0);
-        gi = grab(1);
+        gi = fixed_pos(1, k + 1);
         hne = s_list[min(gi, nhot - 1)];
         hnl = gi < nhot;
       }
@@ -1164,7 +1172,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
       WarmTile<D, WF> tw[NBW];
       int4 ew[NBW];
       bool lw[NBW];
-      int gi = grab(0);
+      int gi = fixed_pos(0, 0);
       int4 ne = s_list[MAX_LIST - 1 - min(gi, nwarm - 1)];
       bool nl = gi < nwarm;
 #pragma unroll
@@ -1173,7 +1181,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
         lw[k] = nl;
         load_warm<D, WF>(p, kvh, uniform(ne.y), lane, wm, tw[k], nl);
         __builtin_amdgcn_sched_barrier(0);
-        gi = grab(0);
+        gi = fixed_pos(0, k + 1);
         ne = s_list[MAX_LIST - 1 - min(gi, nwarm - 1)];
         nl = gi < nwarm;
       }
