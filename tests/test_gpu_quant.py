@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from oracle import codec
-from paged_tierkv_amd import kernels, workloads as W
+from paged_tierkv_amd import _lib, kernels, workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -336,3 +336,51 @@ def test_absmax_promote_bit_exact(device):
         _eq(hot[i, :, :n].cpu().numpy(), exp.numpy(), f"promote {i}")
         assert (hot[i, :, n:].cpu() == 9.0).all()
     assert table[1:6].tolist() == [0, 1, 2, 3, 4] and states[1:6].tolist() == [0] * 5
+
+
+@pytest.mark.parametrize("warm_format", ["absmax_i8", "ref_u8"])
+@pytest.mark.parametrize("bs,dim", [(16, 128), (16, 64), (4, 16), (8, 12), (64, 128), (64, 256)])
+def test_quantize_tokens_equals_demotion_of_staged_tiles(device, warm_format, bs, dim):
+    # Blocks read from the prompt itself: codes, scales and zero points are
+    # the bits the demotion of the same rows staged as tiles gives.  The odd
+    # prompt length puts the rows of head dim 12 at every 8-byte offset, the
+    # last block ends with the prompt, and jobs out of range write nothing.
+    print(f"[quant] tokens {warm_format} bs={bs} dim={dim}", flush=True)
+    g = torch.Generator().manual_seed(bs * 1000 + dim)
+    B, heads, T, slots = 2, 3, 3 * bs + 3, 9
+    k = (torch.randn((B, heads, T, dim), generator=g) * 2).half()
+    v = torch.randn((B, heads, T, dim), generator=g).half()
+    #            in range                                   sequence  token         slot    past the prompt
+    seq = [0, 1, 1, 0, 1,                                   -1, B,    0, 0,         0, 0,   1]
+    tok = [bs, 0, 3 * bs, 2 * bs, 1,                        0, 0,     -1, T,        0, 0,   3 * bs]
+    num = [bs, 1, 3, bs - 1, bs,                            bs, bs,   bs, 1,        bs, bs, 4]
+    dst = [4, 0, 8, 2, 7,                                   1, 1,     3, 3,         -1, slots, 5]
+    live = 5
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=device)
+    code = torch.int8 if warm_format == "absmax_i8" else torch.uint8
+
+    def pools():
+        p = [torch.full((slots, heads, bs, dim), 77, dtype=code, device=device) for _ in range(2)]
+        if warm_format == "absmax_i8":
+            return p + [torch.full((slots, heads), -1.0, device=device), None,
+                        torch.full((slots, heads), -1.0, device=device), None]
+        return p + [torch.full((slots, heads, bs, 1), -1.0, dtype=torch.float16, device=device) for _ in range(4)]
+
+    tiles = [torch.zeros((live, heads, bs, dim), dtype=torch.float16) for _ in range(2)]
+    for i in range(live):
+        for t, x in zip(tiles, (k, v)):
+            t[i, :, :num[i]] = x[seq[i], :, tok[i]: tok[i] + num[i]]
+    want = pools()
+    kernels.demote_to_warm(tiles[0].to(device), tiles[1].to(device), i32(list(range(live))), i32(dst[:live]),
+                           i32(num[:live]), *want, warm_format=warm_format, pad_tail=True)
+    got = pools()
+    P = _lib.ptr
+    kd, vd, js, jt, jd, jn = k.to(device), v.to(device), i32(seq), i32(tok), i32(dst), i32(num)
+    rc = _lib.lib().tierkv_quantize_tokens(P(kd), P(vd), B, T, P(js), P(jt), P(jd), P(jn), len(seq), P(got[0]), P(got[1]),
+                                           slots, P(got[2]), P(got[3]), P(got[4]), P(got[5]),
+                                           kernels.WARM_FORMATS[warm_format], 1, heads, bs, dim, _lib.stream_of(device))
+    _lib.check(rc, "tierkv_quantize_tokens")
+    torch.cuda.synchronize()
+    for name, a, b in zip(("k", "v", "k scale", "k zero", "v scale", "v zero"), got, want):
+        if a is not None:
+            _eq(a.cpu().numpy(), b.cpu().numpy(), name)

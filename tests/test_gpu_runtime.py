@@ -129,6 +129,41 @@ def test_batched_runtime_matches_model(device, warm_format, policy_mode, cold_mo
     assert 0 < m["resident_kv_bytes"] < m["dense_equivalent_bytes"]
 
 
+@pytest.mark.parametrize("batch", [1, 64, 65])
+def test_append_plan_at_its_batch_edges(device, batch):
+    # Up to 64 sequences one wave plans an append, above a whole workgroup:
+    # the first sequences, the last lane and the first sequence of the next
+    # wave, through an open block, a block boundary and a refused append.
+    kv, D, bs, prompt = 1, 64, 16, 21
+    print(f"[runtime] append plan batch={batch}", flush=True)
+    gen = torch.Generator().manual_seed(batch)
+    rt = BatchedTieredKVRuntime(1, batch, kv, D, 64, block_size=bs, hot_fraction=1.0, warm_fraction=0.0,
+                                policy_mode="hot_warm", policy_interval=1000, device=device)
+    orc = BatchedRuntimeOracle(batch, kv, D, bs, rt.max_blocks, rt.hot_slots, rt.warm_slots, "hot_warm", rt.warm_format)
+    k = torch.randn((batch, kv, prompt, D), generator=gen).half()
+    rt.prefill_layer(0, k.to(device), (-k).to(device), block_scores=None)
+    orc.prefill(k.numpy(), (-k).numpy(), np.zeros((batch, 2), np.float32), *rt.budgets(2))
+    q = torch.zeros((batch, kv, 1, D), dtype=torch.float16, device=device)
+    for step in range(18):
+        k1 = torch.randn((batch, kv, 1, D), generator=gen).half()
+        rt.begin_step()
+        rt.decode_layer(0, q, k1.to(device), (-k1).to(device), 1, D ** -0.5)
+        rt.end_step()
+        orc.append(k1.numpy(), (-k1).numpy())
+    rt.check_errors()
+    _compare(rt, orc, "appends")
+    # One full row refuses the append of every sequence.
+    rt.layers[0].nblocks[batch - 1] = rt.max_blocks
+    rt.layers[0].open[batch - 1] = 0
+    before = [x.clone() for x in (rt.layers[0].meta, rt.layers[0].hot_k)]
+    rt.begin_step()
+    rt.decode_layer(0, q, k1.to(device), k1.to(device), 1, D ** -0.5)
+    with pytest.raises(RuntimeError, match="table row is full"):
+        rt.check_errors()
+    rt.layers[0].ctl[2:] = before[0][rt._meta_views["ctl"][0] + 2:][:2]
+    assert torch.equal(rt.layers[0].meta, before[0]) and torch.equal(rt.layers[0].hot_k, before[1])
+
+
 def test_batched_runtime_reports_exhausted_slots(device):
     # A tiny HOT pool: the append that needs a slot it cannot get appends
     # nothing and raises through check_errors; nothing is overwritten.

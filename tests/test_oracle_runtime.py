@@ -23,6 +23,7 @@ import numpy as np
 import pytest
 
 from oracle.runtime import BatchedRuntimeOracle
+from paged_tierkv_amd.runtime import _prefill_tiers, prefill_states
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 CASES = ["runtime_compact_hot_warm", "runtime_compact_hot_warm_cold", "runtime_dense_hot_warm",
@@ -81,3 +82,21 @@ def test_oracle_runtime_follows_reference_trajectory(name):
             _invariants(orc, where)
             checked += 1
     assert checked > 60
+
+
+@pytest.mark.parametrize("mode", ["hot_warm", "hot_warm_cold"])
+@pytest.mark.parametrize("n", [0, 1, 2, 3, 4, 17])
+def test_prefill_tiers_of_many_rows(n, mode):
+    # Every row at once equals the rows one by one: ties, signed zeros,
+    # infinities, a NaN, and budgets from below zero to above the row.
+    rng = np.random.default_rng(n)
+    rows = np.concatenate([rng.random((4, n)), rng.choice([0.0, -0.0, 1.0, np.inf, -np.inf], (6, n)),
+                           np.zeros((1, n))])
+    nan = rows.copy()
+    nan[0, n // 2: n // 2 + 1] = np.nan
+    for scores in (rows, nan):
+        for hot in (-1, 0, 2, 3, 5, n, n + 3):
+            for warm in (-1, 0, 1, 4, n + 1):
+                got = _prefill_tiers(scores, hot, warm, mode)
+                assert got.shape == scores.shape and got.dtype == np.int32
+                assert got.tolist() == [prefill_states(n, r, hot, warm, mode) for r in scores], (hot, warm)
