@@ -32,9 +32,9 @@
 // each, of which about 8 block the VALU, measured with independent streams),
 // 16 exponentials and about 60 other VALU instructions.  Measured against a
 // two-pass kernel whose four waves took 16 queries each and walked all of K
-// together (B x tokens, 32 / 8 heads, D = 128, fp16): 16 x 2048 700 -> 385 us,
-// 16 x 700 134 -> 58, 2 x 300 41 -> 12, 2 x 4096 453 -> 209, 1 x 8192 (two
-// passes) 746 -> 597; 3 x 1001, 32 / 4 heads, D = 64, bf16 163 -> 29 (that
+// together (B x tokens, 32 / 8 heads, D = 128, fp16): 16 x 2048 700 -> 370 us,
+// 16 x 700 134 -> 55, 2 x 300 41 -> 12, 2 x 4096 453 -> 202, 1 x 8192 (two
+// passes) 746 -> 560; 3 x 1001, 32 / 4 heads, D = 64, bf16 163 -> 22 (that
 // kernel ran 192 workgroups there, each a chain of 63 tiles, twice, for 8
 // heads).  Splitting the keys needs no barrier per tile and gives every wave
 // the same number of tiles; eight waves per workgroup at 2048 tokens took
@@ -86,7 +86,7 @@ struct PrefillParams {
   int64_t qs_b, qs_h, qs_t;      // element strides of q [B, H, T, D]
   int64_t ks_b, ks_h, ks_t;      // element strides of k [B, H_kv, T, D]
   float* partial;                // [B, H_kv, nqb, ntiles]
-  int32_t heads, kv_heads, tokens, nqb, ntiles, batch;
+  int32_t heads, kv_heads, tokens, nqb, ntiles, batch, run;
   float scale_log2;
 };
 
@@ -94,6 +94,7 @@ struct PrefillParams {
 // waves' K tiles.  At 8192 tokens one workgroup of four waves would have the
 // CU to itself; two passes with four waves per workgroup keep three there.
 constexpr int PL_ONE_PASS_TILES = 256;
+constexpr int PL_FOUR_WAVES = 128;         // four waves per workgroup up to 2048 tokens
 constexpr float PL_BIG = 0x1p64f;          // a tile sum above it re-bases the row's reference
 
 // Value of lane 16 * (lane / 16) + (lane + N) % 16 (DPP row rotate).
@@ -134,16 +135,18 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
   float* const s_sum = reinterpret_cast<float*>(s_q);                           // [tiles][64 rows] (ONE_PASS)
   const int wg = int(blockIdx.x);
   const int npairs = p.kv_heads * p.batch;
-  int pair, rest;
-  if ((npairs & 7) == 0) {
-    const int slot = wg >> 3;
-    pair = (slot / p.nqb) * 8 + (wg & 7);
-    rest = slot % p.nqb;
-  } else {
-    pair = wg / p.nqb;
-    rest = wg % p.nqb;
-  }
-  const int qb = p.nqb - 1 - rest;
+  // Consecutive workgroups go to the 8 XCDs in turn: with a multiple of 8
+  // pairs, each XCD serves its own.  Its pairs are taken p.run at a time, the
+  // long rows of all of them first.
+  const bool by_xcd = (npairs & 7) == 0;
+  const int slot = by_xcd ? wg >> 3 : wg;
+  const int mine = by_xcd ? npairs >> 3 : npairs;
+  const int set = slot / (p.nqb * p.run);
+  const int width = min(p.run, mine - set * p.run);
+  const int in = slot - set * p.nqb * p.run;
+  const int local = set * p.run + in % width;
+  const int pair = by_xcd ? local * 8 + (wg & 7) : local;
+  const int qb = p.nqb - 1 - in / width;
   const int kvh = pair % p.kv_heads, b = pair / p.kv_heads;
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int n = lane & 15, g = lane >> 4;
@@ -384,8 +387,12 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
 // block's tiles, in a fixed order, / (H * T) / len(blk).  Row r of a kv head
 // holds tiles up to its last query's, QS * r + QS - 1, and exists if its
 // first query lies in the prompt.  One workgroup per (sequence, RED_COLS
-// blocks): RED_COLS neighbouring blocks per row (whole 64-byte segments)
-// and RED_ROWS rows at a time.
+// blocks): RED_COLS neighbouring blocks per row (whole 64-byte segments) and
+// RED_ROWS rows at a time, from the first row that reaches the blocks on, the
+// kv heads' loads four at a time.  Walking all (kv head, row) pairs, half of
+// them above the diagonal, with a division each, took 11.9 us at 16 x 2048
+// (8 kv heads) and 5.0 at 3 x 1001 (4); now 5.1
+// and 3.9.
 constexpr int RED_COLS = 16;
 constexpr int RED_ROWS = 64;
 __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kernel(const float* partial, float* mass,
@@ -399,14 +406,22 @@ __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kerne
   const int tpb = block_size / 16;
   const int t0 = min(blk, nblk - 1) * tpb;
   const int tn = min(tpb, ntiles - t0);
-  const int total = kv_heads * rows;
-  const float* base = partial + int64_t(b) * total * ntiles;
+  const float* base = partial + int64_t(b) * kv_heads * rows * ntiles;
   float acc = 0.f;
-#pragma unroll 4
-  for (int e = int(threadIdx.x) / RED_COLS; e < total; e += RED_ROWS) {
-    const int r = e % rows;
-    const int end = (16 * qs * r < tokens) ? min(t0 + tn, qs * r + qs) : 0;
-    for (int t = t0; t < end; ++t) acc += base[int64_t(e) * ntiles + t];
+  const int first = int(blockIdx.x) * RED_COLS * tpb / qs;
+  for (int r = first + int(threadIdx.x) / RED_COLS; r < rows; r += RED_ROWS) {
+    const int end = min(t0 + tn, qs * r + qs);
+    for (int t = t0; t < end; ++t) {
+      const float* x = base + int64_t(r) * ntiles + t;
+      int h = 0;
+      for (; h + 4 <= kv_heads; h += 4) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = x[int64_t(h + i) * rows * ntiles];
+        acc += (v[0] + v[1]) + (v[2] + v[3]);
+      }
+      for (; h < kv_heads; ++h) acc += x[int64_t(h) * rows * ntiles];
+    }
   }
   acc += shfl_xor_f(acc, 16);
   acc += shfl_xor_f(acc, 32);
@@ -428,7 +443,7 @@ static hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream) {
   const size_t sums = std::max(q, size_t(p.ntiles) * 64 * sizeof(float));
   // Four waves per workgroup while three workgroups fit a CU's LDS (up to 2048
   // tokens); above, the sums leave room for one or two, so eight waves.
-  if (p.ntiles <= 128)
+  if (p.ntiles <= PL_FOUR_WAVES)
     hipLaunchKernelGGL((prefill_block_mass_kernel<D, T, GP, 4, true>), grid, dim3(64 * 4), 4 * tile + sums, stream, p);
   else if (p.ntiles <= PL_ONE_PASS_TILES)
     hipLaunchKernelGGL((prefill_block_mass_kernel<D, T, GP, 8, true>), grid, dim3(64 * 8), 8 * tile + sums, stream, p);
@@ -500,6 +515,20 @@ extern "C" int32_t tierkv_prefill_block_mass(
   const int qs = G == 1 ? 4 : G == 2 ? 2 : 1;    // 16-query blocks per workgroup and partial row
   p.nqb = (p.ntiles + qs - 1) / qs;
   if (int64_t(p.nqb) * num_kv_heads * batch > 0x7fffffff) return fail(TIERKV_ERR_UNSUPPORTED, "prefill grid too large");
+  // Pairs whose rows are dealt together: as many as keep their K within half
+  // of an XCD's L2, so that the short rows come last and fill the end of the
+  // launch.  One pair after the other left its last pair's long rows to the
+  // end: 3 x 1001 (32 / 4 heads, D = 64, 12 pairs) 28.8 us against 21.5,
+  // 4 x 2048 (32 / 8, D = 128) 99 against 91, 16 x 2048 382 against 374.
+  // Above 2048 tokens a workgroup has its CU to itself or makes two passes,
+  // and rows of one length running in step are slower (2 x 4096: 204 us pair
+  // by pair, 213 with two pairs dealt together).
+  const int64_t pair_bytes = int64_t(tokens) * head_dim * 2;
+  const int64_t pairs = int64_t(num_kv_heads) * batch;
+  p.run = p.ntiles > PL_FOUR_WAVES
+              ? 1
+              : int32_t(std::max<int64_t>(1, std::min<int64_t>((int64_t(2) << 20) / pair_bytes,
+                                                               pairs % 8 == 0 ? pairs / 8 : pairs)));
   p.scale_log2 = scaling * 1.4426950408889634f;
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   hipError_t e;
