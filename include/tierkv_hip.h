@@ -113,8 +113,8 @@ TIERKV_API int32_t tierkv_decode_attention(
  * array in the library (one copy per GPU, held until the process ends; its
  * address is taken and the array zeroed on the first call on each device,
  * with that device current, and that first call waits for the fill, so it
- * must not be under stream capture); launches whose
- * tierkv_decode_workspace_bytes exceed 16 MiB fail with TIERKV_ERR_WORKSPACE.
+ * must not be under stream capture); launches that
+ * cannot run in 16 MiB fail with TIERKV_ERR_WORKSPACE.
  * Every call on a GPU shares that GPU's array: calls that overlap on one GPU
  * (different streams, or host threads) race.  Blocks skipped for an
  * out-of-range slot or state set the array's error word, which
@@ -141,7 +141,9 @@ TIERKV_API int32_t tierkv_decode_attention_noalloc(
  * reference. */
 TIERKV_API int32_t tierkv_decode_noalloc_error_word(int32_t clear, int32_t* word);
 
-/* Workspace bytes tierkv_decode_attention needs for this shape. */
+/* Workspace bytes with which tierkv_decode_attention plans freely for this
+ * shape and for every shorter row.  A launch given less takes the best plan
+ * that fits; it is refused only below the bytes of the plain split rule. */
 TIERKV_API int64_t tierkv_decode_workspace_bytes(
     int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t num_blocks,
     int32_t block_size, int32_t head_dim, int32_t with_scores, int32_t splits_hint);
@@ -304,10 +306,11 @@ TIERKV_API int64_t tierkv_runtime_tick_scratch_bytes(int32_t batch, int64_t tabl
  * [B, H_kv, T, D] are fp16 or bf16 with the given element strides (head_dim
  * contiguous, strides multiples of 8, 16-byte aligned); head_dim 64 or 128,
  * GQA group <= 8, block_size a multiple of 16, T <= 32768.  mass is fp32
- * [B, ceil(T / block_size)].  Two MFMA passes over K (log-sum-exp, then
- * block sums); deterministic (fixed reduction order).  workspace: at least
+ * [B, ceil(T / block_size)].  One MFMA pass over K up to 4096 tokens, two
+ * above; deterministic (fixed reduction order).  workspace: at least
  * tierkv_prefill_block_mass_workspace_bytes(B, H_kv, T) bytes, no
- * initialisation needed. */
+ * initialisation needed; with twice as many, short launches of groups above
+ * four heads run as two sets of heads side by side (another summation order). */
 TIERKV_API int64_t tierkv_prefill_block_mass_workspace_bytes(int32_t batch, int32_t num_kv_heads, int32_t tokens);
 TIERKV_API int32_t tierkv_prefill_block_mass(
     const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,

@@ -34,7 +34,7 @@
 // two-pass kernel whose four waves took 16 queries each and walked all of K
 // together (B x tokens, 32 / 8 heads, D = 128, fp16): 16 x 2048 700 -> 370 us,
 // 16 x 700 134 -> 55, 2 x 300 41 -> 12, 2 x 4096 453 -> 202, 1 x 8192 (two
-// passes) 746 -> 560; 3 x 1001, 32 / 4 heads, D = 64, bf16 163 -> 22 (that
+// passes) 746 -> 560; 3 x 1001, 32 / 4 heads, D = 64, bf16 163 -> 20 (that
 // kernel ran 192 workgroups there, each a chain of 63 tiles, twice, for 8
 // heads).  Splitting the keys needs no barrier per tile and gives every wave
 // the same number of tiles; eight waves per workgroup at 2048 tokens took
@@ -85,8 +85,8 @@ struct PrefillParams {
   const void* k;
   int64_t qs_b, qs_h, qs_t;      // element strides of q [B, H, T, D]
   int64_t ks_b, ks_h, ks_t;      // element strides of k [B, H_kv, T, D]
-  float* partial;                // [B, H_kv, nqb, ntiles]
-  int32_t heads, kv_heads, tokens, nqb, ntiles, batch, run;
+  float* partial;                // [B, H_kv, rows, ntiles], rows = nqb * sets
+  int32_t heads, kv_heads, tokens, nqb, ntiles, batch, run, sets;
   float scale_log2;
 };
 
@@ -95,6 +95,7 @@ struct PrefillParams {
 // CU to itself; two passes with four waves per workgroup keep three there.
 constexpr int PL_ONE_PASS_TILES = 256;
 constexpr int PL_FOUR_WAVES = 128;         // four waves per workgroup up to 2048 tokens
+constexpr int TWO_SETS_ROWS = 2048;
 constexpr float PL_BIG = 0x1p64f;          // a tile sum above it re-bases the row's reference
 
 // Value of lane 16 * (lane / 16) + (lane + N) % 16 (DPP row rotate).
@@ -120,8 +121,8 @@ typedef void __attribute__((address_space(3)))* lptr_t;
 
 // GP heads of a kv head's group share a workgroup's rows: slot s is head
 // h0 + s % GP of the group and query block s / GP of the workgroup's 4 / GP
-// blocks of 16 queries; groups of more than GP heads are walked one head set
-// after the other.
+// blocks of 16 queries.  A group of more than GP heads has two head sets: a
+// workgroup each (sets = 2), or one after the other in the same workgroup.
 template <int D, typename T, int GP, int NW, bool ONE_PASS>
 __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillParams p) {
   constexpr int KS = D / 32;                 // MFMA k-steps (one 16-byte chunk per lane each)
@@ -138,15 +139,18 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
   // Consecutive workgroups go to the 8 XCDs in turn: with a multiple of 8
   // pairs, each XCD serves its own.  Its pairs are taken p.run at a time, the
   // long rows of all of them first.
+  const int rows = p.nqb * p.sets;
   const bool by_xcd = (npairs & 7) == 0;
   const int slot = by_xcd ? wg >> 3 : wg;
   const int mine = by_xcd ? npairs >> 3 : npairs;
-  const int set = slot / (p.nqb * p.run);
-  const int width = min(p.run, mine - set * p.run);
-  const int in = slot - set * p.nqb * p.run;
-  const int local = set * p.run + in % width;
+  const int batch0 = slot / (rows * p.run) * p.run;
+  const int width = min(p.run, mine - batch0);
+  const int in = slot - rows * batch0;
+  const int local = batch0 + in % width;
   const int pair = by_xcd ? local * 8 + (wg & 7) : local;
-  const int qb = p.nqb - 1 - in / width;
+  const int row = rows - 1 - in / width;
+  const int first_head = p.sets == 2 ? (row & 1) * GP : 0;
+  const int qb = p.sets == 2 ? row >> 1 : row;
   const int kvh = pair % p.kv_heads, b = pair / p.kv_heads;
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int n = lane & 15, g = lane >> 4;
@@ -156,7 +160,7 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
   const float sl = p.scale_log2;
   const int diag0 = q0 >> 4;                                // the first query block's diagonal tile
   const int last = min(diag0 + QS - 1, (Tn - 1) >> 4);      // the workgroup's last tile
-  float* out = p.partial + (int64_t(pair) * p.nqb + qb) * p.ntiles;
+  float* out = p.partial + (int64_t(pair) * rows + row) * p.ntiles;
 
   // K tiles: this wave's own 16 rows in LDS, filled by loads that go straight
   // there (1 KB each, whole rows).  Chunk c of row r lies at position
@@ -195,13 +199,13 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
     src_tile += NW;
   };
 
-  for (int h0 = 0; h0 < G; h0 += GP) {
+  for (int h0 = first_head; h0 < G; h0 += GP * p.sets) {
     // Q: slot s's 16 rows are staged by wave s like a K tile, in the LDS that
     // holds the tile sums later, and every wave reads its B-operands from
     // there (queries and heads clamped; rows outside the prompt or the group
     // get weight 0 at the end).  Operand-wise loads from memory would have
     // every wave of the workgroup fetch the 64 rows in 64-byte pieces.
-    if (h0 > 0) __syncthreads();                   // the previous head set's sums have been read
+    if (h0 > first_head) __syncthreads();          // the previous head set's sums have been read
 #pragma unroll
     for (int s = w; s < 4; s += NW) {
       const int head = kvh * G + min(h0 + s % GP, G - 1);
@@ -342,7 +346,7 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
       r += row_ror_f<2>(r);
       r += row_ror_f<1>(r);
       const int t = t0 + g * NW;
-      if (n == 0 && t <= last) out[t] = (h0 > 0) ? out[t] + r : r;
+      if (n == 0 && t <= last) out[t] = (h0 > first_head) ? out[t] + r : r;
     };
     if constexpr (ONE_PASS) {
       // Weight of the row in this wave, and this wave's tiles four at a time.
@@ -383,22 +387,21 @@ __global__ __launch_bounds__(64 * NW, 3) void prefill_block_mass_kernel(PrefillP
   }
 }
 
-// mass[b, blk] = sum over the partial rows (kv head, 16 * QS queries) and the
-// block's tiles, in a fixed order, / (H * T) / len(blk).  Row r of a kv head
-// holds tiles up to its last query's, QS * r + QS - 1, and exists if its
-// first query lies in the prompt.  One workgroup per (sequence, RED_COLS
+// mass[b, blk] = sum over the partial rows (kv head, 16 * QS queries, head set)
+// and the block's tiles, in a fixed order, / (H * T) / len(blk).  Row r of a kv
+// head holds tiles up to its last query's, QS * (r / sets) + QS - 1.  One workgroup per (sequence, RED_COLS
 // blocks): RED_COLS neighbouring blocks per row (whole 64-byte segments) and
 // RED_ROWS rows at a time, from the first row that reaches the blocks on, the
 // kv heads' loads four at a time.  Walking all (kv head, row) pairs, half of
 // them above the diagonal, with a division each, took 11.9 us at 16 x 2048
-// (8 kv heads) and 5.0 at 3 x 1001 (4); now 5.1
-// and 3.9.
+// (8 kv heads) and 5.0 at 3 x 1001 (4); now 5.1 and 3.9.
 constexpr int RED_COLS = 16;
 constexpr int RED_ROWS = 64;
 __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kernel(const float* partial, float* mass,
-                                                                                   int kv_heads, int rows, int qs,
-                                                                                   int ntiles, int heads, int tokens,
-                                                                                   int block_size, int nblk) {
+                                                                                   int kv_heads, int rows, int sets,
+                                                                                   int qs, int ntiles, int heads,
+                                                                                   int tokens, int block_size,
+                                                                                   int nblk) {
   __shared__ float s_part[RED_COLS * RED_ROWS / 64][RED_COLS];
   const int b = blockIdx.y;
   const int col = threadIdx.x % RED_COLS;
@@ -408,9 +411,9 @@ __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kerne
   const int tn = min(tpb, ntiles - t0);
   const float* base = partial + int64_t(b) * kv_heads * rows * ntiles;
   float acc = 0.f;
-  const int first = int(blockIdx.x) * RED_COLS * tpb / qs;
+  const int first = int(blockIdx.x) * RED_COLS * tpb / qs * sets;
   for (int r = first + int(threadIdx.x) / RED_COLS; r < rows; r += RED_ROWS) {
-    const int end = min(t0 + tn, qs * r + qs);
+    const int end = min(t0 + tn, qs * (r >> (sets - 1)) + qs);
     for (int t = t0; t < end; ++t) {
       const float* x = base + int64_t(r) * ntiles + t;
       int h = 0;
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kerne
 
 template <int D, typename T, int GP>
 static hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream) {
-  const dim3 grid(unsigned(int64_t(p.nqb) * p.kv_heads * p.batch));
+  const dim3 grid(unsigned(int64_t(p.nqb) * p.sets * p.kv_heads * p.batch));
   const size_t tile = 16 * D * 2;
   const size_t q = 64 * D * 2;   // the tile sums take its place
   const size_t sums = std::max(q, size_t(p.ntiles) * 64 * sizeof(float));
@@ -514,7 +517,17 @@ extern "C" int32_t tierkv_prefill_block_mass(
   p.batch = batch;
   const int qs = G == 1 ? 4 : G == 2 ? 2 : 1;    // 16-query blocks per workgroup and partial row
   p.nqb = (p.ntiles + qs - 1) / qs;
-  if (int64_t(p.nqb) * num_kv_heads * batch > 0x7fffffff) return fail(TIERKV_ERR_UNSUPPORTED, "prefill grid too large");
+  const int64_t grid = int64_t(p.nqb) * num_kv_heads * batch;
+  if (grid > 0x7fffffff) return fail(TIERKV_ERR_UNSUPPORTED, "prefill grid too large");
+  // The two head sets of a group above four heads run side by side, each
+  // workgroup half as long, when the workspace holds a partial row for each
+  // and the launch has no more than eight rows per CU: 1 x 1000 (8 / 1 heads,
+  // D = 128) 22.1 -> 14.4 us, 3 x 1001 (32 / 4, D = 64) 21.6 -> 19.7,
+  // 4 x 2048 (32 / 4, D = 128) 99.7 -> 97.7, 1 x 8192 626 -> 585.  Longer
+  // launches are full either way and read twice the partials: 16 x 700
+  // (32 / 4, D = 64, 2816 rows) 41.7 -> 42.8, 2 x 4096 (64 / 8, D = 128, 4096
+  // rows) 409 -> 421.
+  p.sets = (G > 4 && grid <= TWO_SETS_ROWS && workspace_bytes >= 2 * need) ? 2 : 1;
   // Pairs whose rows are dealt together: as many as keep their K within half
   // of an XCD's L2, so that the short rows come last and fill the end of the
   // launch.  One pair after the other left its last pair's long rows to the
@@ -541,6 +554,6 @@ extern "C" int32_t tierkv_prefill_block_mass(
   const int nblk = (tokens + block_size - 1) / block_size;
   hipLaunchKernelGGL(prefill_mass_reduce_kernel, dim3((nblk + RED_COLS - 1) / RED_COLS, batch),
                      dim3(RED_COLS * RED_ROWS), 0, stream, p.partial, mass, num_kv_heads,
-                     p.nqb, qs, p.ntiles, num_heads, tokens, block_size, nblk);
+                     p.nqb * p.sets, p.sets, qs, p.ntiles, num_heads, tokens, block_size, nblk);
   return check_launch("prefill_mass_reduce_kernel");
 }

@@ -204,6 +204,8 @@ def prefill_block_mass(query_states: torch.Tensor, key_states: torch.Tensor, blo
         raise ValueError("key states do not match the query geometry.")
     kv_heads = int(k.shape[1])
     need = int(lib.tierkv_prefill_block_mass_workspace_bytes(batch, kv_heads, tokens))
+    if heads > 4 * kv_heads and batch * kv_heads * ((tokens + 15) // 16) <= 2048:
+        need *= 2      # the shapes whose two sets of heads run side by side
     # One scratch buffer per (device, stream): launches on one stream are
     # ordered; launches on different streams may overlap and never share it.
     key = (q.device.index, _lib.stream_of(q.device))

@@ -77,6 +77,10 @@ def test_prefill_block_mass_agrees_with_compute_block_scores(device):
     (1, 5, 1, 530, 128, torch.bfloat16),     # two head sets, the second with three idle slots
     (1, 2, 2, 4096, 64, torch.float16),      # the last one-pass length
     (1, 2, 1, 4100, 64, torch.float16),      # two passes, partial last tile
+    (128, 5, 1, 250, 64, torch.float16),     # 2048 rows: the last launch with head sets side by side
+    (129, 5, 1, 250, 64, torch.bfloat16),    # the first with one after the other
+    (3, 8, 2, 1001, 64, torch.float16),      # six pairs dealt together
+    (1, 18, 18, 2048, 128, torch.float16),   # 18 pairs dealt four at a time, the last two by themselves
     (9, 1, 1, 65, 128, torch.float16),       # pairs not a multiple of the XCDs, one row past a 64-query block
 ])
 def test_prefill_block_mass_edges(device, B, H, Hkv, T, D, dtype):
