@@ -443,8 +443,8 @@ def run_prefill(args, device):
     """The prefill block-score kernel (tierkv_prefill_block_mass: per-block
     causal attention mass of one layer's prefill, without materialised
     probabilities) at C5's prefill shape.  One step = one call for the whole
-    batch.  Algorithmic FLOPs: two passes of q . k over the causal pairs,
-    2 * 2 * B * H * T(T+1)/2 * D."""
+    batch.  Algorithmic FLOPs: q . k once over the causal pairs,
+    2 * B * H * T(T+1)/2 * D (the result needs no second product)."""
     import torch
 
     from paged_tierkv_amd import kernels
@@ -474,7 +474,7 @@ def run_prefill(args, device):
     e1.record()
     torch.cuda.synchronize()
     sec = e0.elapsed_time(e1) / 1e3 / steps
-    flops = 2 * 2 * B * H * (T * (T + 1) // 2) * D
+    flops = 2 * B * H * (T * (T + 1) // 2) * D
     tf = flops / sec / 1e12
     log(f"[prefill] {sec * 1e3:.3f} ms per call, {tf:.1f} TFLOP/s ({tf / PEAK_MFMA_F16_TFLOPS:.1%} of the fp16 peak)")
     cpu = None
@@ -491,7 +491,7 @@ def run_prefill(args, device):
             t0 = time.perf_counter()
             oracle_mass(qn, kn, scaling, 16)
             per = time.perf_counter() - t0
-        sflops = 2 * 2 * G * (T * (T + 1) // 2) * D
+        sflops = 2 * G * (T * (T + 1) // 2) * D
         cpu = {"value": round(sflops / per / 1e12, 6), "unit": "TFLOP/s", "cores": 1, "kind": "port",
                "sample": f"one sequence, one kv head ({G} q heads) of the batch, {per:.1f} s "
                          "(oracle NumPy float64 probabilities, single thread)"}
