@@ -143,8 +143,15 @@ TIERKV_API int32_t tierkv_decode_noalloc_error_word(int32_t clear, int32_t* word
 
 /* Workspace bytes with which tierkv_decode_attention plans freely for this
  * shape and for every shorter row.  A launch given less takes the best plan
- * that fits; it is refused only below the bytes of the plain split rule. */
+ * that fits; it is refused only below tierkv_decode_workspace_least_bytes. */
 TIERKV_API int64_t tierkv_decode_workspace_bytes(
+    int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t num_blocks,
+    int32_t block_size, int32_t head_dim, int32_t with_scores, int32_t splits_hint);
+
+/* The fewest workspace bytes that tierkv_decode_attention accepts for this
+ * shape: those of enough splits to put about 2048 waves on the chip, or of
+ * the hint. */
+TIERKV_API int64_t tierkv_decode_workspace_least_bytes(
     int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t num_blocks,
     int32_t block_size, int32_t head_dim, int32_t with_scores, int32_t splits_hint);
 

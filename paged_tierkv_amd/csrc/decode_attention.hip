@@ -1893,6 +1893,13 @@ static int reported_splits(int64_t units, int num_blocks, int groups, int splits
   return splits;
 }
 
+// Bytes of the smallest workspace that a launch is accepted with.
+static int64_t least_workspace(int batch, int num_heads, int kv_heads, int num_blocks, int block_size, int head_dim,
+                               bool scores, int splits_hint) {
+  const int splits = required_splits(int64_t(batch) * kv_heads, num_blocks, num_heads / kv_heads, splits_hint);
+  return ws_layout(batch, num_heads, kv_heads, num_blocks, block_size, head_dim, scores, splits).total;
+}
+
 template <int D, int WF, bool SC, bool CZ, typename QT, int NW>
 static void launch_nw(const DecodeParams& p, bool long_rows, int grid, hipStream_t stream) {
   size_t shmem = size_t(NW) * p.groups * D * sizeof(float);
@@ -1969,6 +1976,15 @@ extern "C" int64_t tierkv_decode_workspace_bytes(int32_t batch, int32_t num_head
   return ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, with_scores != 0, splits).total;
 }
 
+extern "C" int64_t tierkv_decode_workspace_least_bytes(int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                                                       int32_t num_blocks, int32_t block_size, int32_t head_dim,
+                                                       int32_t with_scores, int32_t splits_hint) {
+  if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_blocks <= 0 || block_size <= 0 || head_dim <= 0)
+    return -1;
+  return least_workspace(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, with_scores != 0,
+                         hint_splits(splits_hint));
+}
+
 // Every argument check of tierkv_decode_attention, before anything is
 // launched (tierkv_decode_step runs it ahead of its token write, so a refused
 // step changes nothing on the device).
@@ -2009,8 +2025,9 @@ int32_t tierkv::decode_check_args(
   const bool scores = score_sums != nullptr;
   const int groups = num_heads / num_kv_heads;
   const int splits = required_splits(int64_t(batch) * num_kv_heads, num_blocks, groups, splits_hint);
-  const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores, splits);
-  if (workspace_bytes < wl.total) return fail(TIERKV_ERR_WORKSPACE, "workspace too small");
+  if (workspace_bytes < least_workspace(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores,
+                                        splits_hint))
+    return fail(TIERKV_ERR_WORKSPACE, "workspace too small");
   if (fast_path_ok(block_size, head_dim, groups) && table_stride <= 0x7fffffff) {
     const bool aligned = aligned16(hot_k) && aligned16(hot_v) && aligned16(warm_k) && aligned16(warm_v) &&
                          aligned16(query);
@@ -2240,13 +2257,8 @@ extern "C" int32_t tierkv_decode_attention_noalloc(
   clear_error();
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
   // Invalid shapes are left to tierkv_decode_attention's checks.
-  int64_t need = 0;
-  if (batch > 0 && num_heads > 0 && num_kv_heads > 0 && num_blocks > 0 && block_size > 0 && head_dim > 0) {
-    const int splits = required_splits(int64_t(batch) * num_kv_heads, num_blocks, num_heads / num_kv_heads,
-                                       hint_splits(splits_hint));
-    need = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, score_sums != nullptr,
-                     splits).total;
-  }
+  const int64_t need = tierkv_decode_workspace_least_bytes(batch, num_heads, num_kv_heads, num_blocks, block_size,
+                                                           head_dim, score_sums != nullptr, splits_hint);
   if (need > STATIC_SCRATCH_BYTES)
     return fail(TIERKV_ERR_WORKSPACE, "tierkv_decode_attention_noalloc: this launch needs " + std::to_string(need) +
                                           " bytes of scratch; the allocation-free entry point holds " +

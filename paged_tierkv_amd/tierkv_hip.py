@@ -69,12 +69,13 @@ class DecodeWorkspace:
     one stream, or otherwise ordered).
 
     ``growable=False`` fixes the buffer for the workspace's lifetime: a call
-    that needs more raises instead of reallocating.  Captured graphs hold the
+    whose plan would use more takes a plan that fits, and one that cannot run
+    in it raises instead of reallocating.  Captured graphs hold the
     buffer's address, so a workspace used under capture must be sized before
     the capture (``DecodeWorkspace.for_shape``); the first launch bound to a
     workspace under capture fixes it, so that no later eager launch can free
     memory a graph replays on.  A growable workspace replaces its buffer when
-    a call needs more bytes; the error flags set in the old buffer are carried
+    a call's plan uses more bytes; the error flags set in the old buffer are carried
     into the new one on the device (no host sync), and the old buffer is
     recorded on every stream that used it before it is dropped, so the
     caching allocator reuses it only after their queued work.  The reference
@@ -123,9 +124,13 @@ class DecodeWorkspace:
     def _capturing(self) -> bool:
         return self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
-    def reserve(self, nbytes: int) -> None:
+    def reserve(self, nbytes: int, least: int | None = None) -> None:
+        """Make room for a launch that plans freely with ``nbytes`` bytes and
+        can run in ``least`` (default: ``nbytes``).  A buffer that may not be
+        replaced (fixed, or under capture) only has to hold ``least``."""
+        least = nbytes if least is None else least
         capturing = self._capturing()
-        if nbytes <= self.nbytes:
+        if nbytes <= self.nbytes or (least <= self.nbytes and (capturing or not self.growable)):
             if capturing:
                 self.growable = False   # a graph holds this buffer's address from now on
             return
@@ -134,7 +139,7 @@ class DecodeWorkspace:
                                "(a DecodeWorkspace sized before the capture), or run the launch once eagerly "
                                "on this stream first.")
         if not self.growable:
-            raise RuntimeError(f"decode workspace holds {self.nbytes} bytes, the launch needs {int(nbytes)}: "
+            raise RuntimeError(f"decode workspace holds {self.nbytes} bytes, the launch needs {int(least)}: "
                                "size the fixed workspace for the largest launch (DecodeWorkspace.for_shape).")
         new = torch.zeros(int(nbytes), dtype=torch.uint8, device=self.device)
         new[:4].view(torch.int32).bitwise_or_(self.buf[:4].view(torch.int32))
@@ -151,6 +156,16 @@ class DecodeWorkspace:
         if word and clear:
             self.buf[:4].zero_()
         return word
+
+
+def launch_bytes(lib, *shape) -> tuple[int, int]:
+    """``DecodeWorkspace.reserve``'s arguments for a launch of ``shape``
+    (batch, heads, kv heads, blocks, block size, head dim, with scores, splits
+    hint): the bytes it plans freely with and the fewest it is accepted with."""
+    need = lib.tierkv_decode_workspace_bytes(*shape)
+    if need < 0:
+        raise ValueError("invalid decode geometry.")
+    return need, lib.tierkv_decode_workspace_least_bytes(*shape)
 
 
 _LIVE: "weakref.WeakSet[DecodeWorkspace]" = weakref.WeakSet()
@@ -327,12 +342,10 @@ def _rebind(lib, query_states, statics, num_blocks, num_key_value_groups, scalin
     if need is None:
         # tail: hot_k, hot_v, hot_slots, warm_k, warm_v, warm_slots, k_scale, k_zero, v_scale, v_zero,
         # fmt, cold, batch, heads, kv_heads, block_size, head_dim, scaling, splits hint
-        need = needs[n] = lib.tierkv_decode_workspace_bytes(batch, num_heads, tail[14], n, tail[15], head_dim,
-                                                            int(return_scores), tail[18])
-        if need < 0:
-            raise ValueError("invalid decode geometry.")
+        need = needs[n] = launch_bytes(lib, batch, num_heads, tail[14], n, tail[15], head_dim, int(return_scores),
+                                       tail[18])
     ws = stream_workspace(device)
-    ws.reserve(need)
+    ws.reserve(*need)
     args = ((_lib.ptr(query), dtype_code, _lib.ptr(out), _lib.ptr(score_sums)) + mid + (n,) + tail +
             (ws.data_ptr(), ws.nbytes))
     return args, out, score_sums, ws, batched
@@ -469,10 +482,8 @@ def _bind(
         raise ValueError("splits must be a non-negative split factor.")
     if default_deterministic() if deterministic is None else deterministic:
         splits_hint |= _lib.DECODE_DETERMINISTIC
-    need = lib.tierkv_decode_workspace_bytes(batch, num_heads, kv_heads, int(num_blocks), block_size,
-                                             head_dim, int(return_scores), splits_hint)
-    if need < 0:
-        raise ValueError("invalid decode geometry.")
+    need = launch_bytes(lib, batch, num_heads, kv_heads, int(num_blocks), block_size, head_dim, int(return_scores),
+                        splits_hint)
     if isinstance(workspace, str):
         if workspace != NOALLOC:
             raise ValueError(f"workspace must be a DecodeWorkspace, None or {NOALLOC!r}.")
@@ -481,13 +492,13 @@ def _bind(
         ws = workspace
         ws.note_stream(torch.cuda.current_stream(device))
     elif prepared:
-        ws = DecodeWorkspace(device, need, growable=False)
+        ws = DecodeWorkspace(device, need[0], growable=False)
     else:
         ws = stream_workspace(device)
     if ws is not None:
         if ws.device != device:
             raise ValueError("the decode workspace lives on another device.")
-        ws.reserve(need)
+        ws.reserve(*need)
         if prepared and ws.growable:
             raise ValueError("a prepared decode needs a fixed workspace (DecodeWorkspace(..., growable=False)).")
     args = (

@@ -1392,12 +1392,10 @@ class CompactTieredKVTensorPool(_PoolBase):
         need = needs.get(n)
         lib = _lib.lib()
         if need is None:
-            need = needs[n] = lib.tierkv_decode_workspace_bytes(st.batch, st.num_heads, st.num_kv_heads, n,
-                                                                st.block_size, st.head_dim, 0, st.splits_hint)
-            if need < 0:
-                return None
+            need = needs[n] = tierkv_hip.launch_bytes(lib, st.batch, st.num_heads, st.num_kv_heads, n, st.block_size,
+                                                      st.head_dim, 0, st.splits_hint)
         ws = tierkv_hip.stream_workspace(self.device)
-        ws.reserve(need)
+        ws.reserve(*need)
         out = torch.empty((1, 1, st.num_heads, st.head_dim), device=self.device, dtype=query_states.dtype)
         # Host state first, as the general path records it before launching.
         self._blocks[physical_idx] = _Block(HOT_STATE, b.slot, pos + 1)

@@ -578,3 +578,28 @@ def test_smallest_accepted_workspace(device):
     assert call(smallest - 1) == _lib.TIERKV_ERR_WORKSPACE
     torch.cuda.synchronize()
     assert int(plan.out.count_nonzero()) == 0
+
+
+def test_fixed_workspace_of_a_larger_batch(device):
+    """A fixed workspace sized for 128 sequences has no room for the split
+    partials that 33 sequences would use: they run unsplit in it, eagerly, in
+    a prepared launch and under capture."""
+    from paged_tierkv_amd.tierkv_hip import DecodeWorkspace, PreparedDecode
+
+    case = W.make_tiered_case("ws_batch", 33, 16, 8, 64, 144, 16, 80, seed=4)
+    ws = DecodeWorkspace.for_shape(device, 128, 16, 8, 144, 64, return_scores=False)
+    assert ws.nbytes < DecodeWorkspace.bytes_for(33, 16, 8, 144, 64, return_scores=False)
+    before = ws.data_ptr()
+    want, _ = _check(case, "absmax_i8", device, cold_mode="masked", seqs=[0, 16, 32], workspace=ws)
+    plan = PreparedDecode(**to_gpu_inputs(case, oracle_warm(case, "absmax_i8"), device), cold_mode="masked",
+                          workspace=ws)
+    assert_close(plan.launch()[0].float().cpu().numpy(), want.float().cpu().numpy(), what="prepared launch")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.launch()
+    for _ in range(3):
+        plan.out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(plan.out.float().cpu().numpy(), want.float().cpu().numpy(), what="replay")
+    assert ws.data_ptr() == before and ws.error_word() == 0

@@ -5,6 +5,8 @@
 * A growable workspace carries its error flags into the new buffer.
 * A workspace first bound under stream capture becomes fixed, so a later,
   larger eager launch cannot free memory a captured graph replays on.
+* A workspace that cannot be replaced serves every launch the library accepts
+  it for, also where the launch's free plan would use more.
 * The batched runtime sizes its fixed workspace once, for ``max_blocks``
   with score sums; every smaller launch of the same geometry (any block
   count, with or without scores) fits in it, so nothing it launches can ask
@@ -16,7 +18,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from paged_tierkv_amd.tierkv_hip import DecodeWorkspace
+from paged_tierkv_amd import _lib
+from paged_tierkv_amd.tierkv_hip import DecodeWorkspace, launch_bytes
 
 
 def test_fixed_workspace_never_replaces_its_buffer():
@@ -107,3 +110,64 @@ def test_reported_bytes_cover_every_shorter_row(batch, heads, kv, dim, scores):
         need = DecodeWorkspace.bytes_for(batch, heads, kv, nb, dim, return_scores=scores)
         assert need >= last, (nb, need, last)
         last = need
+
+
+def _plain_rule_bytes(batch, heads, kv, nb, dim, scores, splits=0):
+    """Workspace of the plain split rule: about 2048 waves on the chip, at
+    least four tiles per wave, rows under 12 tiles per wave whole."""
+    units, nw = batch * kv, 8 if heads // kv <= 8 else 4
+    if not splits:
+        splits = min(max(1, -(-2048 // (units * nw))), max(1, nb // (4 * nw)))
+        if nb < 12 * nw:
+            splits = 1
+    splits = max(1, min(max(splits, -(-nb // 511)), nb))
+    up = lambda x: -(-x // 256) * 256
+    partials = up(batch * heads * splits * dim * 4) + up(batch * heads * splits * 2 * 4) if splits > 1 else 0
+    return 256 + (1 << 16) * 4 + partials + (up(batch * heads * nb * 2 * 4) if scores else 0)
+
+
+@pytest.mark.parametrize("heads,kv,dim", [(32, 8, 128), (32, 4, 64), (16, 16, 64), (64, 4, 128)])
+def test_least_bytes_are_the_plain_split_rules(heads, kv, dim):
+    lib = _lib.lib()
+    for batch in (1, 2, 7, 31, 32, 33, 40, 64, 65, 128):
+        for nb in (1, 9, 33, 95, 96, 144, 256, 511, 512, 1100, 2048):
+            for scores in (0, 1):
+                for splits in (0, 1, 3, 8):
+                    full, least = launch_bytes(lib, batch, heads, kv, nb, 16, dim, scores, splits)
+                    assert least == _plain_rule_bytes(batch, heads, kv, nb, dim, scores, splits), (batch, nb, splits)
+                    assert least <= full
+    assert lib.tierkv_decode_workspace_least_bytes(0, 32, 8, 256, 16, 128, 0, 0) < 0
+
+
+@pytest.mark.parametrize("batch", [32, 33, 40, 48, 63, 64])
+def test_fixed_workspace_serves_smaller_batches(batch, monkeypatch):
+    """A workspace sized for a large batch holds no split partials, where a
+    smaller batch's free plan would split: it is served unsplit, eagerly in a
+    fixed workspace and under capture in a growable one."""
+    shape = (batch, 32, 8, 256, 16, 128, 0, 0)
+    full, least = launch_bytes(_lib.lib(), *shape)
+    ws = DecodeWorkspace.for_shape("cpu", 128, 32, 8, 256, 128, return_scores=False)
+    assert least <= ws.nbytes < full
+    before = ws.data_ptr()
+    ws.reserve(full, least)
+    assert ws.data_ptr() == before and ws.nbytes < full
+    warmed = DecodeWorkspace("cpu")
+    warmed.reserve(*launch_bytes(_lib.lib(), 128, *shape[1:]))
+    before = warmed.data_ptr()
+    monkeypatch.setattr(DecodeWorkspace, "_capturing", lambda self: True)
+    warmed.reserve(full, least)
+    assert warmed.data_ptr() == before and not warmed.growable
+    monkeypatch.setattr(DecodeWorkspace, "_capturing", lambda self: False)
+    warmed.reserve(full, least)         # fixed by the capture
+    assert warmed.data_ptr() == before
+    grown = DecodeWorkspace("cpu", least)
+    grown.reserve(full, least)          # growable: room for the free plan
+    assert grown.nbytes == full
+
+
+def test_workspace_below_the_least_bytes_is_refused():
+    full, least = launch_bytes(_lib.lib(), 16, 32, 8, 256, 16, 128, 1, 0)
+    assert least < full
+    DecodeWorkspace("cpu", least, growable=False).reserve(full, least)
+    with pytest.raises(RuntimeError, match=f"needs {least}:"):
+        DecodeWorkspace("cpu", least - 1, growable=False).reserve(full, least)
