@@ -106,6 +106,23 @@ def _prefill_tiers(scores: np.ndarray, hot_budget: int, warm_budget: int, policy
     return out
 
 
+def _score_rows(block_scores, batch: int, n: int) -> np.ndarray:
+    """``prefill_layer``'s scores as float64 rows of n blocks: one row shared
+    by every sequence (None: the proxy, or a 1-D sequence), or one each."""
+    if block_scores is None:
+        scores = np.array(recency_scores(n), dtype=np.float64)
+    else:
+        scores = torch.as_tensor(block_scores, dtype=torch.float32).detach().cpu().numpy().astype(np.float64)
+    if scores.ndim == 1:
+        scores = scores[None]
+    elif scores.shape[0] < batch:
+        raise IndexError("block_scores needs one row per sequence.")
+    if n > 2 and scores.shape[1] < n - 1:
+        raise IndexError("block_scores needs one score per candidate block.")
+    scores = np.pad(scores, ((0, 0), (0, max(n - scores.shape[1], 0))))   # the last block is no candidate
+    return scores[:batch, :n]
+
+
 def _strided_f16(t: torch.Tensor) -> torch.Tensor:
     """fp16 tensor whose head dimension is contiguous, with strides that are
     multiples of 8 elements and a 16-byte aligned start (copied otherwise)."""
@@ -297,18 +314,8 @@ class BatchedTieredKVRuntime:
         k = key_states.to(torch.float16).contiguous()
         v = value_states.to(torch.float16).contiguous()
         hot_b, warm_b = self.budgets(n)
-        if block_scores is None:
-            scores = np.array(recency_scores(n), dtype=np.float64)
-        else:
-            scores = torch.as_tensor(block_scores, dtype=torch.float32).cpu().numpy().astype(np.float64)
-        if scores.ndim == 1:
-            scores = scores[None]
-        elif scores.shape[0] < B:
-            raise IndexError("block_scores needs one row per sequence.")
-        if n > 2 and scores.shape[1] < n - 1:
-            raise IndexError("block_scores needs one score per candidate block.")
-        scores = np.pad(scores, ((0, 0), (0, max(n - scores.shape[1], 0))))   # the last block is no candidate
-        tiers = np.broadcast_to(_prefill_tiers(scores[:B, :n], hot_b, warm_b, self.policy_mode), (B, n))
+        tiers = np.broadcast_to(_prefill_tiers(_score_rows(block_scores, B, n), hot_b, warm_b, self.policy_mode),
+                                (B, n))
         bs = self.block_size
         first = np.arange(n, dtype=np.int32) * bs               # each block's first token
         count = np.minimum(T - first, bs).astype(np.int32)

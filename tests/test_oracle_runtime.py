@@ -21,9 +21,10 @@ import os
 
 import numpy as np
 import pytest
+import torch
 
 from oracle.runtime import BatchedRuntimeOracle
-from paged_tierkv_amd.runtime import _prefill_tiers, prefill_states
+from paged_tierkv_amd.runtime import _prefill_tiers, _score_rows, prefill_states, recency_scores
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 CASES = ["runtime_compact_hot_warm", "runtime_compact_hot_warm_cold", "runtime_dense_hot_warm",
@@ -100,3 +101,27 @@ def test_prefill_tiers_of_many_rows(n, mode):
                 got = _prefill_tiers(scores, hot, warm, mode)
                 assert got.shape == scores.shape and got.dtype == np.int32
                 assert got.tolist() == [prefill_states(n, r, hot, warm, mode) for r in scores], (hot, warm)
+
+
+@pytest.mark.parametrize("make", [
+    lambda x: x.tolist(), lambda x: x, lambda x: x.numpy(), lambda x: x.double(), lambda x: x.bfloat16(),
+    lambda x: x.clone().requires_grad_(), lambda x: (x.clone().requires_grad_() * 2.0) / 2.0,
+    lambda x: x.t().contiguous().t() if x.ndim == 2 else x[:, None].expand(-1, 2).contiguous()[:, 0],
+], ids=["list", "tensor", "numpy", "double", "bf16", "leaf", "graph", "strided"])
+def test_prefill_scores_of_every_kind(make):
+    # Scores come as lists, arrays or tensors, of a graph or not, shared by
+    # the sequences or one row each; the last block's may be missing.
+    torch.manual_seed(0)
+    n, batch = 7, 3
+    for shape in ((n,), (n - 1,), (n + 2,), (batch, n), (batch + 1, n - 1)):
+        given = make(torch.rand(shape))
+        want = torch.as_tensor(given, dtype=torch.float32).tolist()
+        got = _score_rows(given, batch, n)
+        rows = [want] if len(shape) == 1 else want[:batch]
+        assert got.shape == (len(rows), n) and got.dtype == np.float64
+        for g, w in zip(got.tolist(), rows):
+            assert g == (w + [0.0])[:n]
+    assert _score_rows(None, batch, n).tolist() == [recency_scores(n)]
+    for short in (torch.rand(n - 2), torch.rand(batch, n - 2), torch.rand(batch - 1, n)):
+        with pytest.raises(IndexError):
+            _score_rows(short, batch, n)
