@@ -603,3 +603,33 @@ def test_fixed_workspace_of_a_larger_batch(device):
         torch.cuda.synchronize()
         assert_close(plan.out.float().cpu().numpy(), want.float().cpu().numpy(), what="replay")
     assert ws.data_ptr() == before and ws.error_word() == 0
+
+
+@pytest.mark.parametrize("batch,kv,groups,dim,nb", [(2, 8, 4, 128, 144), (6, 4, 1, 128, 86), (3, 2, 8, 64, 400)])
+def test_deterministic_bits_and_the_workspace_size(device, batch, kv, groups, dim, nb):
+    """A deterministic launch gives one result in every workspace with room
+    for its plan, and one other in every smaller one that is accepted."""
+    from paged_tierkv_amd import _lib
+    from paged_tierkv_amd.tierkv_hip import PreparedDecode, launch_bytes
+
+    case = W.make_tiered_case(f"det_ws_{nb}", batch, kv * groups, kv, dim, nb, nb // 8, nb // 2, seed=nb)
+    lib = _lib.lib()
+    args = to_gpu_inputs(case, oracle_warm(case, "absmax_i8"), device)
+    plan = PreparedDecode(**args, cold_mode="masked", deterministic=True)
+    full, least = launch_bytes(lib, batch, kv * groups, kv, nb, 16, dim, 0, 0)
+    assert plan.workspace.nbytes == full > least
+    want = plan.launch()[0].clone()
+    ws = torch.zeros(2 * full, dtype=torch.uint8, device=device)
+    outs = []
+    for size in sorted({least + (full - least) * i // 12 for i in range(13)} | {full + 1, 2 * full}):
+        plan.out.zero_()
+        rc = lib.tierkv_decode_attention(*plan._args[:-2], ws.data_ptr(), size, _lib.stream_of(device))
+        assert rc == _lib.TIERKV_OK
+        torch.cuda.synchronize()
+        assert_close(plan.out.float().cpu().numpy(), want.float().cpu().numpy(), what=f"{size} bytes")
+        outs.append(plan.out.clone())
+        if size >= full:
+            assert torch.equal(plan.out, want)
+    kinds = [torch.equal(o, want) for o in outs]
+    assert kinds == sorted(kinds), "a smaller workspace gave the full one's bits, a larger one not"
+    assert all(torch.equal(o, outs[0]) for o, k in zip(outs, kinds) if not k)
