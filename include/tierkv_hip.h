@@ -319,9 +319,13 @@ TIERKV_API int64_t tierkv_runtime_tick_scratch_bytes(int32_t batch, int64_t tabl
  * [B, ceil(T / block_size)].  One MFMA pass over K up to 4096 tokens, two
  * above; deterministic (fixed reduction order).  workspace: at least
  * tierkv_prefill_block_mass_workspace_bytes(B, H_kv, T) bytes, no
- * initialisation needed; with twice as many, short launches of groups above
- * four heads run as two sets of heads side by side (another summation order). */
+ * initialisation needed; with tierkv_prefill_block_mass_full_workspace_bytes,
+ * which are twice as many for short launches of groups above four heads, those
+ * run as two sets of heads side by side (another summation order; results
+ * follow from the shape and from which of the two sizes is reached). */
 TIERKV_API int64_t tierkv_prefill_block_mass_workspace_bytes(int32_t batch, int32_t num_kv_heads, int32_t tokens);
+TIERKV_API int64_t tierkv_prefill_block_mass_full_workspace_bytes(int32_t batch, int32_t num_heads,
+                                                                  int32_t num_kv_heads, int32_t tokens);
 TIERKV_API int32_t tierkv_prefill_block_mass(
     const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
     const void* k, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t, int32_t dtype,

@@ -141,6 +141,7 @@ SIGNATURES = {
         c_int32, _P, _P, c_int64,
         c_int32, c_int32, c_int32, _P]),
     "tierkv_prefill_block_mass_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32]),
+    "tierkv_prefill_block_mass_full_workspace_bytes": (c_int64, [c_int32] * 4),
     "tierkv_prefill_block_mass": (c_int32, [
         _P, c_int64, c_int64, c_int64,
         _P, c_int64, c_int64, c_int64, c_int32,

@@ -438,6 +438,18 @@ __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kerne
   }
 }
 
+// The two head sets of a group above four heads run side by side, each
+// workgroup half as long, when the launch has no more than eight rows per CU
+// (and the workspace holds a partial row for each): 1 x 1000 (8 / 1 heads,
+// D = 128) 22.1 -> 14.4 us, 3 x 1001 (32 / 4, D = 64) 21.6 -> 19.0,
+// 4 x 2048 (32 / 4, D = 128) 99.7 -> 97.7, 1 x 8192 626 -> 585.  Longer
+// launches are full either way and read twice the partials: 16 x 700
+// (32 / 4, D = 64, 2816 rows) 41.7 -> 42.8, 2 x 4096 (64 / 8, D = 128, 4096
+// rows) 409 -> 421.
+static bool head_sets_side_by_side(int groups, int64_t pairs, int64_t ntiles) {
+  return groups > 4 && pairs * ntiles <= TWO_SETS_ROWS;
+}
+
 template <int D, typename T, int GP>
 static hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream) {
   const dim3 grid(unsigned(int64_t(p.nqb) * p.sets * p.kv_heads * p.batch));
@@ -474,6 +486,14 @@ extern "C" int64_t tierkv_prefill_block_mass_workspace_bytes(int32_t batch, int3
   const int64_t rows = (tokens + 63) / 64 * 4;
   const int64_t ntiles = (tokens + 15) / 16;
   return int64_t(batch) * num_kv_heads * rows * ntiles * 4;
+}
+
+extern "C" int64_t tierkv_prefill_block_mass_full_workspace_bytes(int32_t batch, int32_t num_heads,
+                                                                  int32_t num_kv_heads, int32_t tokens) {
+  const int64_t need = tierkv_prefill_block_mass_workspace_bytes(batch, num_kv_heads, tokens);
+  if (need < 0 || num_heads <= 0) return -1;
+  const bool two = head_sets_side_by_side(num_heads / num_kv_heads, int64_t(batch) * num_kv_heads, (tokens + 15) / 16);
+  return two ? 2 * need : need;
 }
 
 extern "C" int32_t tierkv_prefill_block_mass(
@@ -519,15 +539,8 @@ extern "C" int32_t tierkv_prefill_block_mass(
   p.nqb = (p.ntiles + qs - 1) / qs;
   const int64_t grid = int64_t(p.nqb) * num_kv_heads * batch;
   if (grid > 0x7fffffff) return fail(TIERKV_ERR_UNSUPPORTED, "prefill grid too large");
-  // The two head sets of a group above four heads run side by side, each
-  // workgroup half as long, when the workspace holds a partial row for each
-  // and the launch has no more than eight rows per CU: 1 x 1000 (8 / 1 heads,
-  // D = 128) 22.1 -> 14.4 us, 3 x 1001 (32 / 4, D = 64) 21.6 -> 19.7,
-  // 4 x 2048 (32 / 4, D = 128) 99.7 -> 97.7, 1 x 8192 626 -> 585.  Longer
-  // launches are full either way and read twice the partials: 16 x 700
-  // (32 / 4, D = 64, 2816 rows) 41.7 -> 42.8, 2 x 4096 (64 / 8, D = 128, 4096
-  // rows) 409 -> 421.
-  p.sets = (G > 4 && grid <= TWO_SETS_ROWS && workspace_bytes >= 2 * need) ? 2 : 1;
+  const int64_t pairs = int64_t(num_kv_heads) * batch;
+  p.sets = (head_sets_side_by_side(G, pairs, p.ntiles) && workspace_bytes >= 2 * need) ? 2 : 1;
   // Pairs whose rows are dealt together: as many as keep their K within half
   // of an XCD's L2, so that the short rows come last and fill the end of the
   // launch.  One pair after the other left its last pair's long rows to the
@@ -537,7 +550,6 @@ extern "C" int32_t tierkv_prefill_block_mass(
   // and rows of one length running in step are slower (2 x 4096: 204 us pair
   // by pair, 213 with two pairs dealt together).
   const int64_t pair_bytes = int64_t(tokens) * head_dim * 2;
-  const int64_t pairs = int64_t(num_kv_heads) * batch;
   p.run = p.ntiles > PL_FOUR_WAVES
               ? 1
               : int32_t(std::max<int64_t>(1, std::min<int64_t>((int64_t(2) << 20) / pair_bytes,

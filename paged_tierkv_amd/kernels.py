@@ -203,11 +203,11 @@ def prefill_block_mass(query_states: torch.Tensor, key_states: torch.Tensor, blo
     if k.shape[0] != batch or k.shape[2] != tokens or k.shape[3] != dim:
         raise ValueError("key states do not match the query geometry.")
     kv_heads = int(k.shape[1])
-    need = int(lib.tierkv_prefill_block_mass_workspace_bytes(batch, kv_heads, tokens))
-    if heads > 4 * kv_heads and batch * kv_heads * ((tokens + 15) // 16) <= 2048:
-        need *= 2      # the shapes whose two sets of heads run side by side
+    need = int(lib.tierkv_prefill_block_mass_full_workspace_bytes(batch, heads, kv_heads, tokens))
     # One scratch buffer per (device, stream): launches on one stream are
     # ordered; launches on different streams may overlap and never share it.
+    # The call passes what this shape needs, not what the buffer holds, so its
+    # summation order does not depend on earlier calls.
     key = (q.device.index, _lib.stream_of(q.device))
     ws = _prefill_ws.get(key)
     if ws is None or ws.numel() < need:
@@ -218,6 +218,6 @@ def prefill_block_mass(query_states: torch.Tensor, key_states: torch.Tensor, blo
     rc = lib.tierkv_prefill_block_mass(
         _lib.ptr(q), q.stride(0), q.stride(1), q.stride(2), _lib.ptr(k), k.stride(0), k.stride(1), k.stride(2),
         _lib.DTYPE_BF16 if q.dtype == torch.bfloat16 else _lib.DTYPE_F16, _lib.ptr(out), batch, heads, kv_heads,
-        tokens, dim, int(block_size), float(scaling), _lib.ptr(ws), int(ws.numel()), _lib.stream_of(q.device))
+        tokens, dim, int(block_size), float(scaling), _lib.ptr(ws), need, _lib.stream_of(q.device))
     _lib.check(rc, "tierkv_prefill_block_mass")
     return out

@@ -132,3 +132,17 @@ def test_decode_step_rejects_bad_counts_without_gpu():
     st.n_jobs, st.n_pairs = 1, 0   # a write job with no source or pool pointers
     assert lib.tierkv_decode_step(ctypes.byref(st), None) == _lib.TIERKV_ERR_INVALID
     assert "null" in _lib.last_error()
+
+
+@pytest.mark.parametrize("batch,heads,kv,tokens,two", [
+    (1, 8, 1, 1000, True), (128, 5, 1, 250, True), (129, 5, 1, 250, False), (1, 5, 1, 32768, True),
+    (2, 40, 8, 2048, True), (2, 40, 8, 2049, False), (1, 4, 1, 16, False), (3, 64, 16, 1, False), (3, 64, 8, 1, True),
+])
+def test_prefill_full_workspace_holds_two_head_sets(batch, heads, kv, tokens, two):
+    """Groups above four heads take twice the bytes in launches of at most
+    2048 rows of 16 queries, every other shape the least bytes."""
+    lib = _lib.lib()
+    least = lib.tierkv_prefill_block_mass_workspace_bytes(batch, kv, tokens)
+    assert lib.tierkv_prefill_block_mass_full_workspace_bytes(batch, heads, kv, tokens) == (2 if two else 1) * least > 0
+    assert lib.tierkv_prefill_block_mass_full_workspace_bytes(batch, 0, kv, tokens) < 0
+    assert lib.tierkv_prefill_block_mass_full_workspace_bytes(batch, heads, 0, tokens) < 0

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from oracle.policy import prefill_block_mass as oracle_mass
-from paged_tierkv_amd import kernels, tierkv_policy as tp
+from paged_tierkv_amd import _lib, kernels, tierkv_policy as tp
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,33 @@ def test_prefill_block_mass_growing_logits(device, T, growth):
     got = kernels.prefill_block_mass(q.to(device), k.to(device), 16, 64 ** -0.5).cpu().numpy()
     want = oracle_mass(q.float().numpy(), k.float().numpy(), 64 ** -0.5, 16)
     np.testing.assert_allclose(got, want, rtol=5e-4, atol=1e-9)
+
+
+def _mass_in(q, k, scaling, nbytes):
+    """Block masses (16-token blocks) in a workspace of nbytes of a larger buffer."""
+    (B, H, T, D), Hkv = q.shape, k.shape[1]
+    out = torch.full((B, -(-T // 16)), -1.0, dtype=torch.float32, device=q.device)
+    ws = torch.full((nbytes + 4096,), 255, dtype=torch.uint8, device=q.device)   # NaN where it is read unwritten
+    rc = _lib.lib().tierkv_prefill_block_mass(
+        _lib.ptr(q), *q.stride()[:3], _lib.ptr(k), *k.stride()[:3],
+        _lib.DTYPE_BF16 if q.dtype == torch.bfloat16 else _lib.DTYPE_F16, _lib.ptr(out), B, H, Hkv, T, D, 16, scaling,
+        _lib.ptr(ws), nbytes, _lib.stream_of(q.device))
+    _lib.check(rc, "tierkv_prefill_block_mass")
+    torch.cuda.synchronize()
+    assert bool((ws[nbytes:] == 255).all()), "wrote past the workspace"
+    return out
+
+
+def test_prefill_scores_do_not_depend_on_earlier_calls(device):
+    """Launches too long for head sets side by side give the same bits before
+    and after a call that made the shared scratch larger."""
+    g = torch.Generator().manual_seed(2)
+    q = torch.randn((129, 5, 250, 64), generator=g).half().to(device)
+    k = torch.randn((129, 1, 250, 64), generator=g).half().to(device)
+    lib = _lib.lib()
+    least = lib.tierkv_prefill_block_mass_workspace_bytes(129, 1, 250)
+    assert lib.tierkv_prefill_block_mass_full_workspace_bytes(129, 5, 1, 250) == least
+    want = _mass_in(q, k, 0.125, least)
+    kernels.prefill_block_mass(torch.cat([q] * 3), torch.cat([k] * 3), 16, 0.125)
+    assert torch.equal(kernels.prefill_block_mass(q, k, 16, 0.125), want)
+    assert torch.equal(_mass_in(q, k, 0.125, 4 * least), want)
