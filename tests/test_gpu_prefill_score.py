@@ -124,6 +124,40 @@ def _mass_in(q, k, scaling, nbytes):
     return out
 
 
+@pytest.mark.parametrize("G,T,D,dtype,growth", [
+    (5, 2100, 64, torch.float16, 0.0),       # eight waves, the second head set with three idle slots
+    (8, 2100, 128, torch.bfloat16, 0.0),
+    (6, 4090, 128, torch.float16, 0.0),      # the last one-pass length in tiles, a partial last tile
+    (5, 4100, 128, torch.bfloat16, 0.0),     # two passes
+    (8, 4100, 64, torch.float16, 0.0),
+    (7, 2500, 64, torch.float16, 30.0),      # references raised with eight waves and two head sets
+    (7, 4300, 64, torch.float16, 30.0),
+])
+def test_prefill_head_sets_beyond_2048_tokens(device, G, T, D, dtype, growth):
+    """Groups above four heads in the eight-wave and the two-pass kernels, the
+    two head sets one after the other and side by side (the two workspace
+    sizes), and through the wrapper, which takes the second."""
+    print(f"[prefill-sets] G={G} T={T} D={D} {dtype} growth={growth}", flush=True)
+    g = torch.Generator().manual_seed(T + G)
+    q = torch.randn((1, G, T, D), generator=g).to(dtype)
+    k = torch.randn((1, 1, T, D), generator=g)
+    if growth:
+        k = k * (torch.linspace(0.1, 1.0, T) * growth)[None, None, :, None]
+    k = k.to(dtype)
+    want = oracle_mass(q.float().numpy(), k.float().numpy(), D ** -0.5, 16)
+    lib = _lib.lib()
+    least = lib.tierkv_prefill_block_mass_workspace_bytes(1, 1, T)
+    full = lib.tierkv_prefill_block_mass_full_workspace_bytes(1, G, 1, T)
+    assert full == 2 * least
+    qd, kd = q.to(device), k.to(device)
+    one, two = (_mass_in(qd, kd, D ** -0.5, n) for n in (least, full))
+    # Logits of several hundred carry a few roundings of 300 * 2^-24 in the exponent.
+    tol = 5e-4 if growth else 1e-4
+    for got in (one, two):
+        np.testing.assert_allclose(got.cpu().numpy(), want, rtol=tol, atol=1e-9)
+    assert torch.equal(kernels.prefill_block_mass(qd, kd, 16, D ** -0.5), two)
+
+
 def test_prefill_scores_do_not_depend_on_earlier_calls(device):
     """Launches too long for head sets side by side give the same bits before
     and after a call that made the shared scratch larger."""
