@@ -51,20 +51,6 @@
 
 namespace tierkv {
 
-// Where a score launch stages each block's (max, sum) per head:
-//   STAGE_LDS_BLOCK LDS [G][num_blocks] by logical block (unsplit launches),
-//                   finalised by the workgroup itself;
-//   STAGE_LDS_LIST  LDS [G][MAX_LIST] by list position, copied to the
-//                   workspace [B][H][num_blocks] at the end of the workgroup
-//                   (split launches);
-//   STAGE_GLOBAL    the workspace, written per tile (rows too long for LDS).
-// The workspace stages are finalised by finalize_scores_kernel, launched
-// after the decode kernel: one workgroup per (sequence, q head) row spreads
-// that work over the chip, where a unit's last workgroup would read every
-// staged pair of the unit and write its whole score rows from one CU.
-constexpr int STAGE_GLOBAL = 0;
-constexpr int STAGE_LDS_BLOCK = 1;
-constexpr int STAGE_LDS_LIST = 2;
 constexpr float PBOOST = 64.f;     // P is scaled by 2^6 before its fp16 cast
 constexpr float LAZY_T = 8.f;      // log2 headroom of the running maximum
 constexpr float FOLD_MAX = 2.f;    // WARM V scales above this are applied to V
@@ -98,7 +84,7 @@ struct DecodeParams {
   float scaling;
   int32_t splits;
   uint32_t split_magic;   // ceil(2^32 / splits) when num_blocks * splits < 2^32, else 0
-  int32_t lds_stage;      // where score statistics are staged (STAGE_* below)
+  int32_t lds_stage;      // where score statistics are staged (STAGE_*, decode_plan.h)
   int32_t deterministic;  // host only: fixed tile shares per wave (TIERKV_DECODE_DETERMINISTIC)
   float* ws_acc;      // [units][splits][G][D]
   float* ws_ml;       // [units][splits][G][2]
@@ -753,7 +739,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void tiered_decode_kernel(
   // Blocks of this sequence: the per-sequence count is loaded together with
   // the first row chunk and applied afterwards.
   const int nb_ld = a_seq_nblocks ? a_seq_nblocks[b] : a_num_blocks;
-  // Per-block score statistics (max, sum) per head (STAGE_* modes above).
+  // Per-block score statistics (max, sum) per head (STAGE_* modes).
   // Nothing the list build does depends on the stage mode, a kernel argument
   // outside the preloaded ones whose load would hold the build up.  A block
   // that no tile will visit gets an entry too (stage_blank), so the staged
@@ -1737,9 +1723,7 @@ __global__ __launch_bounds__(64) void decode_generic_kernel(DecodeParams p) {
 
 template <int D, int WF, bool SC, bool CZ, typename QT, int NW>
 static void launch_nw(const DecodeParams& p, bool long_rows, int grid, hipStream_t stream) {
-  size_t shmem = size_t(NW) * p.groups * D * sizeof(float);
-  if (SC && p.lds_stage == STAGE_LDS_BLOCK) shmem += size_t(p.groups) * p.num_blocks * 2 * sizeof(float);
-  if (SC && p.lds_stage == STAGE_LDS_LIST) shmem += size_t(p.groups) * MAX_LIST * 2 * sizeof(float);
+  const size_t shmem = size_t(dynamic_lds(NW, p.groups, D, p.num_blocks, p.lds_stage));
   const int32_t stride = int32_t(p.table_stride);
   const bool xcd_seq = p.splits == 1 && p.batch % 8 == 0;   // see tiered_decode_kernel
   const int32_t kvh_splits = int32_t(uint32_t(p.kv_heads) | (uint32_t(p.splits) << 16) |
@@ -1909,8 +1893,8 @@ extern "C" int32_t tierkv_decode_attention(
   const bool scores = score_sums != nullptr;
   const bool fast = fast_path_ok(block_size, head_dim, num_heads / num_kv_heads) && table_stride <= 0x7fffffff;
   // (alignment and launch limits: decode_check_args)
-  const Plan pl = fast ? plan_launch(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores,
-                                     splits_hint, det, workspace_bytes)
+  const Plan pl = fast ? plan_launch(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, warm_format,
+                                     scores, splits_hint, det, workspace_bytes)
                        : Plan{1, 1};
   const WsLayout wl = ws_layout(batch, num_heads, num_kv_heads, num_blocks, block_size, head_dim, scores, pl.splits);
 
@@ -1955,19 +1939,7 @@ extern "C" int32_t tierkv_decode_attention(
   if (fast) {
     p.splits = pl.splits;
     p.split_magic = 0;
-    // Unsplit score launches keep the per-block statistics in LDS (up to
-    // MAX_LDS_STAGE bytes per workgroup) and finalise them in the workgroup;
-    // split ones stage them in LDS by list position and copy them to the
-    // workspace, where finalize_scores_kernel reads them.
-    p.lds_stage = STAGE_GLOBAL;
-    if (scores) {
-      const int64_t pair = 2 * int64_t(sizeof(float));
-      if (pl.splits == 1 && int64_t(p.groups) * num_blocks * pair <= MAX_LDS_STAGE) {
-        p.lds_stage = STAGE_LDS_BLOCK;
-      } else if (pl.splits > 1 && int64_t(p.groups) * MAX_LIST * pair <= MAX_LDS_STAGE) {
-        p.lds_stage = STAGE_LDS_LIST;
-      }
-    }
+    p.lds_stage = score_stage(scores, p.groups, num_blocks, pl.splits);
     if (pl.splits > 1 && int64_t(num_blocks) * pl.splits < (int64_t(1) << 32))
       p.split_magic = uint32_t(((uint64_t(1) << 32) + uint64_t(pl.splits) - 1) / uint64_t(pl.splits));
     // Split launches go out in chunks of whole sequences, at most

@@ -5,6 +5,8 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "tierkv_hip.h"
+
 namespace tierkv {
 
 constexpr int FBS = 16;            // tokens per block on the fast path
@@ -13,6 +15,20 @@ constexpr int MAX_WAVES = 8;
 constexpr int PRE_CHUNKS = 4;      // table-row chunks loaded together by the list build
 constexpr int MERGE_UNROLL = 8;    // split partials loaded together by the merge
 constexpr int MAX_LDS_STAGE = 48 * 1024;   // bytes of per-block score statistics kept in LDS
+// Where a score launch stages each block's (max, sum) per head:
+//   STAGE_LDS_BLOCK LDS [G][num_blocks] by logical block (unsplit launches),
+//                   finalised by the workgroup itself;
+//   STAGE_LDS_LIST  LDS [G][MAX_LIST] by list position, copied to the
+//                   workspace [B][H][num_blocks] at the end of the workgroup
+//                   (split launches);
+//   STAGE_GLOBAL    the workspace, written per tile (rows too long for LDS).
+// The workspace stages are finalised by finalize_scores_kernel, launched
+// after the decode kernel: one workgroup per (sequence, q head) row spreads
+// that work over the chip, where a unit's last workgroup would read every
+// staged pair of the unit and write its whole score rows from one CU.
+constexpr int STAGE_GLOBAL = 0;
+constexpr int STAGE_LDS_BLOCK = 1;
+constexpr int STAGE_LDS_LIST = 2;
 constexpr int MAX_SPLIT_UNITS = 1 << 16;   // units per launch when a unit is split
 
 struct Plan {
@@ -45,45 +61,104 @@ inline int required_splits(int64_t units, int num_blocks, int groups, int splits
   return int(std::max<int64_t>(1, std::min<int64_t>(splits, num_blocks)));
 }
 
+// The stage of a launch: unsplit score launches keep the statistics in LDS
+// (up to MAX_LDS_STAGE bytes per workgroup) and finalise them in the workgroup;
+// split ones stage them in LDS by list position.
+inline int score_stage(bool scores, int groups, int num_blocks, int splits) {
+  const int64_t pair = 2 * int64_t(sizeof(float));
+  if (!scores) return STAGE_GLOBAL;
+  if (splits == 1) return int64_t(groups) * num_blocks * pair <= MAX_LDS_STAGE ? STAGE_LDS_BLOCK : STAGE_GLOBAL;
+  return groups * MAX_LIST * pair <= MAX_LDS_STAGE ? STAGE_LDS_LIST : STAGE_GLOBAL;
+}
+
+// LDS of a workgroup: the wave accumulators and the stage, beside the kernel's
+// own arrays (the list and the waves' counts and sums).
+constexpr int STATIC_LDS = 9728;
+inline int64_t dynamic_lds(int nw, int groups, int head_dim, int num_blocks, int stage) {
+  int64_t bytes = int64_t(nw) * groups * head_dim * int64_t(sizeof(float));
+  if (stage == STAGE_LDS_BLOCK) bytes += int64_t(groups) * num_blocks * 2 * int64_t(sizeof(float));
+  if (stage == STAGE_LDS_LIST) bytes += int64_t(groups) * MAX_LIST * 2 * int64_t(sizeof(float));
+  return bytes;
+}
+
+// Waves of the decode kernel that a SIMD's 512 vector registers hold: 206 to
+// 230 registers at head_dim 128, at head_dim 64 127 in the absmax format and
+// 132 to 151 in the reference format or with score sums.
+inline int waves_per_simd(int head_dim, int warm_format, bool scores) {
+  if (head_dim == 128) return 2;
+  return warm_format == TIERKV_WARM_ABSMAX_I8 && !scores ? 4 : 3;
+}
+
+// Workgroups of nw waves that run together on a CU (four SIMDs, 160 KB of
+// LDS).  A score launch of a large group at head_dim 64 is held to fewer by
+// its statistics than by registers.
+inline int64_t workgroups_per_cu(int num_blocks, int groups, int head_dim, int warm_format, bool scores, int nw,
+                                 int s) {
+  const int64_t by_registers = 4 * waves_per_simd(head_dim, warm_format, scores) / nw;
+  const int64_t lds = STATIC_LDS + dynamic_lds(nw, groups, head_dim, num_blocks,
+                                               score_stage(scores, groups, num_blocks, s));
+  return std::max<int64_t>(1, std::min(by_registers, 160 * 1024 / lds));
+}
+
 // Expected time (us, less the launch itself) of a launch with nw waves per
-// workgroup and s splits per unit.  A CU moves about 26 B/ns whether one or
-// two workgroups and four or eight waves stream on it, so what counts is how
-// many workgroups the busiest CU gets, how many of them run together (by
-// registers: one of eight waves at head_dim 128, two at 64; twice as many of
-// four), and each pass's fixed part (list build, first loads, wave merge).
-// A split adds its publication, arrival and merge, and with score sums the
-// finalisation launch.  The constants are a fit to 6,192 timings (16
-// unit counts from 4 to 1024, ten row lengths from 9 to 2048 blocks, up to 12
-// split counts, both wave counts and head dims, with and without score sums;
-// 10 % HOT, 60 % WARM): over these shapes the plan chosen by it is on average
-// 1 % slower than the fastest measured one, where aiming at 2048 waves with
-// eight per workgroup was 15 % slower (head_dim 64: 9 %, with score sums 17 %;
-// up to 2.1x: 248 units made 496 workgroups of 256 that fit at a time).
-inline double plan_cost(int64_t units, int num_blocks, int head_dim, bool scores, int nw, int s) {
-  const double per_block = head_dim == 64 ? 0.038 : 0.091;   // a block's tiles at a CU's rate
-  const double per_wave = 0.231;                             // a block's round trips in one wave
-  const double fixed = nw == 4 ? 6.0 : 6.4;
-  const int64_t room = (head_dim == 64 ? 2 : 1) * (nw == 4 ? 2 : 1);
+// workgroup and s splits per unit: what counts is how many workgroups the
+// busiest CU gets, how many of them run together (workgroups_per_cu), their
+// blocks' time, and what is fixed in each pass (list build, first loads, wave
+// merge) and in each split (publication, arrival, merge, and with score sums
+// the finalisation launch).
+// The constants are one least-squares fit (of the logarithm) to 17,589
+// timings: 1,336 shapes of 1 to 1024 units, 8 to 2048 blocks, GQA groups 1 to
+// 16, both head dims and formats, with and without score sums, 5 to 30 % HOT
+// and 40 to 65 % WARM, each with both wave counts and up to 13 split counts,
+// in graphs over four layers' buffers.  The plan chosen by it is on average
+// 0.6 % slower than the fastest measured one (fitted on either half and
+// checked on the other, too); the plain rule of required_splits with the most
+// waves is 15 % slower, up to 3.5 times (units * s just above what runs at
+// once).  1 shape in 50 is more than 3 % slower than with it (worst
+// 1.14 times).
+inline double plan_cost(int64_t units, int num_blocks, int groups, int head_dim, int warm_format, bool scores, int nw,
+                        int s) {
+  // A block's tiles in a workgroup, alone or sharing its CU: 256 units, D =
+  // 128, 10 % HOT, 60 % WARM (3.3 KB per block) take 25.6 us at 144 blocks and
+  // 58.3 at 400, 0.128 per block (26 B/ns).  Four waves alone at D = 64 have
+  // too few loads in flight (64 units of 256 blocks: 25.1 us, 18.6 with eight).
+  const double per_block = head_dim == 64 ? 0.060 : 0.125;
+  const double alone = head_dim == 64 && nw == 4 ? 1.42 : 1.0;
+  const double fixed = nw == 4 ? 3.98 : 5.17;
+  const int64_t room = workgroups_per_cu(num_blocks, groups, head_dim, warm_format, scores, nw, s);
   const int64_t on_cu = (units * s + 255) / 256;
   const int64_t passes = (on_cu + room - 1) / room;
-  const double refill = room == 1 ? 1.0 : nw == 4 ? 1.8 : 0.3;   // a further pass against the first
-  const double blocks = double(num_blocks) / s;
-  // One pass with so many workgroups together on the CU.  Four waves alone
-  // stream 3 % slower than eight (256 units of 1024 blocks: 145 against 141
-  // us), three workgroups of four where four fit (head_dim 64) 8 % (632
-  // units of 496 blocks: 88.8 against 81.8).
-  auto pass = [&](int64_t together) {
-    const double slower = nw == 4 && together == 1 && s == 1 ? 1.03 : nw == 4 && room == 4 && together == 3 ? 1.08 : 1.0;
-    return std::max(slower * per_block * blocks * together, per_wave * blocks / nw);
-  };
+  const double refill = room == 1 ? 1.44 : nw == 4 ? 1.81 : 1.21;   // a further pass's fixed part against the first's
+  auto pass = [&](int64_t together) { return per_block * num_blocks / s * std::max(double(together), alone); };
   double t = fixed + (passes - 1) * (fixed * refill + pass(std::min(on_cu, room))) +
              pass(on_cu - (passes - 1) * room);
-  if (s > 1)
-    t += 1.7 + (scores ? (nw == 4 ? 4.9 : 4.1) : 0.0) + 1.5 * ((s + MERGE_UNROLL - 1) / MERGE_UNROLL) +
-         0.3 * (std::min(on_cu, room) - 1);
-  // Rows longer than one pass of the list build (with score sums, the blanks
-  // of the later passes are written one by one).
-  t += ((num_blocks - 1) / (PRE_CHUNKS * nw * 64)) * (scores ? 3.5 : 1.0);
+  const int threads = 64 * nw, elements = groups * head_dim;
+  if (s > 1) {
+    // Publication and merge: MERGE_UNROLL splits and one or two elements per
+    // thread and round trip; workgroups on one CU publish in turn (64 units of
+    // 256 blocks, D = 64, G = 4: 14.5 us in two splits of eight waves, 12.0 in
+    // four, 14.7 in five, where two share a CU).
+    const int rounds = (s + MERGE_UNROLL - 1) / MERGE_UNROLL;
+    const int per_trip = elements > threads ? 2 * threads : threads;
+    t += 0.59 * rounds + 0.96 * rounds * ((elements + per_trip - 1) / per_trip) +
+         0.61 * ((elements + threads - 1) / threads) + 1.52 * (std::min(on_cu, room) - 1);
+  }
+  // Score sums: the workgroup's own waves, a head or a part of one each (8
+  // units of 64 blocks unsplit, G = 4: 10.9 -> 13.8 us with eight waves, 11.5
+  // -> 15.4 with four), or a finalisation launch of a workgroup per (sequence,
+  // head) row (the same in eight splits 8.8 -> 13.4 us; 1024 rows, 128 units
+  // of 256 blocks at D = 64 in two splits: 29.7 us, 23.2 unsplit).
+  if (scores && score_stage(scores, groups, num_blocks, s) == STAGE_LDS_BLOCK)
+    t += 1.9 * (((groups <= 8 ? 8 / groups * groups : groups) + nw - 1) / nw);
+  else if (scores)
+    t += 4.27 + 5.06 * double(units * groups) / 512;
+  // The list build of rows beyond one chunk (256 units, D = 128, four waves
+  // against eight: 0.5 us less at 256 blocks, 0.6 more at 320), and beyond one
+  // pass (32 units of 2048 blocks in eight splits: 30.7 us with eight waves,
+  // one pass; 32.1 with four, two), where the blanks of the score sums are
+  // written one by one.
+  if (num_blocks > threads) t += 1.09;
+  t += ((num_blocks - 1) / (PRE_CHUNKS * threads)) * (scores ? 4.9 : 1.5);
   return t;
 }
 
@@ -141,7 +216,7 @@ inline int64_t least_workspace(int batch, int num_heads, int kv_heads, int num_b
 // in every workspace with room for it, and in every smaller one the plan of
 // the smallest (not the best that fits, which would change with each size).
 inline Plan plan_launch(int batch, int num_heads, int kv_heads, int num_blocks, int block_size, int head_dim,
-                        bool scores, int splits_hint, bool deterministic, int64_t workspace_bytes) {
+                        int warm_format, bool scores, int splits_hint, bool deterministic, int64_t workspace_bytes) {
   const int groups = num_heads / kv_heads;
   const int64_t units = int64_t(batch) * kv_heads;
   auto bytes = [&](int s) {
@@ -153,7 +228,7 @@ inline Plan plan_launch(int batch, int num_heads, int kv_heads, int num_blocks, 
     auto consider = [&](int s) {
       for (int nw = 8; nw >= 4; nw -= 4) {
         if (nw == 8 && groups > 8) continue;
-        const double c = plan_cost(units, num_blocks, head_dim, scores, nw, s);
+        const double c = plan_cost(units, num_blocks, groups, head_dim, warm_format, scores, nw, s);
         if (c < best_cost) {
           best_cost = c;
           best = Plan{nw, s};
