@@ -151,7 +151,19 @@ class LayerStorage:
     hot_free: torch.Tensor    # [hot capacity] free-slot stack
     warm_free: torch.Tensor   # [warm capacity]
     ctl: torch.Tensor         # [4] hot_top, warm_top, error bits, last append applied
-    meta: torch.Tensor        # the int32 buffer the eight tensors above are views of
+    meta: torch.Tensor | None = None   # the int32 buffer the eight tensors above are views of
+
+    def load(self, flat: torch.Tensor, views: dict) -> None:
+        """Overwrite the int32 tensors from ``flat``, which holds each at
+        ``views[name]`` = (start, size, shape): one copy while they are the
+        views of ``meta``, else (a caller has put its own tensors in their
+        place) one by one."""
+        m = self.meta
+        if m is not None and all(getattr(self, n).data_ptr() == m.data_ptr() + 4 * at for n, (at, _, _) in views.items()):
+            m.copy_(flat)
+            return
+        for name, (at, size, shape) in views.items():
+            getattr(self, name).copy_(flat[at: at + size].view(shape))
 
 
 class BatchedTieredKVRuntime:
@@ -367,7 +379,7 @@ class BatchedTieredKVRuntime:
                                             _lib.ptr(st.v_zero), kernels.WARM_FORMATS[self.warm_format], 1,
                                             kv, bs, d, stream)
             _lib.check(rc, "tierkv_quantize_tokens")
-        st.meta.copy_(dev[:m])
+        st.load(dev[:m], self._meta_views)
         self._blocks[layer] = n
         self._open_tokens[layer] = 0
         if layer == self.num_layers - 1:

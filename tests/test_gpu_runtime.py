@@ -236,3 +236,24 @@ def test_fused_rope_append_is_bit_exact(device):
         _lib.ptr(st.ctl), kv, bs, D, _lib.stream_of(device))
     _lib.check(rc)
     assert torch.equal(q_rot, q_ref.contiguous())
+
+
+def test_prefill_fills_tensors_put_in_place_of_a_layers_own(device):
+    """A caller may put its own int32 tensors into a layer (a restored table):
+    the next prefill fills those, and decode reads them."""
+    B, kv, D, bs, prompt = 2, 2, 64, 16, 100
+    gen = torch.Generator().manual_seed(3)
+    k, v, q, k1, v1 = (torch.randn((B, kv, n, D), generator=gen).half().to(device) for n in (prompt, prompt, 1, 1, 1))
+    outs = []
+    for own in (False, True):
+        rt = BatchedTieredKVRuntime(1, B, kv, D, 160, block_size=bs, device=device)
+        st = rt.layers[0]
+        if own:
+            for name in ("table", "states", "lengths", "nblocks", "open", "hot_free", "warm_free", "ctl"):
+                setattr(st, name, torch.full_like(getattr(st, name), 0))
+        rt.prefill_layer(0, k, v)
+        rt.begin_step()
+        outs.append(rt.decode_layer(0, q, k1, v1, 1, D ** -0.5).clone())
+        rt.end_step()
+        rt.check_errors()
+    assert torch.equal(*outs) and bool(outs[0].abs().sum() > 0)

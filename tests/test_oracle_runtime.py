@@ -24,7 +24,7 @@ import pytest
 import torch
 
 from oracle.runtime import BatchedRuntimeOracle
-from paged_tierkv_amd.runtime import _prefill_tiers, _score_rows, prefill_states, recency_scores
+from paged_tierkv_amd.runtime import LayerStorage, _prefill_tiers, _score_rows, prefill_states, recency_scores
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 CASES = ["runtime_compact_hot_warm", "runtime_compact_hot_warm_cold", "runtime_dense_hot_warm",
@@ -125,3 +125,23 @@ def test_prefill_scores_of_every_kind(make):
     for short in (torch.rand(n - 2), torch.rand(batch, n - 2), torch.rand(batch - 1, n)):
         with pytest.raises(IndexError):
             _score_rows(short, batch, n)
+
+
+def test_layer_tensors_replaced_by_the_caller_are_loaded():
+    # A prefill fills the tensors the layer holds, whether they are still the
+    # views of its one buffer or the caller's own (a restored table).
+    views = {"table": (0, 6, (2, 3)), "states": (64, 6, (2, 3)), "lengths": (128, 6, (2, 3)), "nblocks": (192, 2, (2,)),
+             "open": (256, 2, (2,)), "hot_free": (320, 4, (4,)), "warm_free": (384, 5, (5,)), "ctl": (448, 4, (4,))}
+    flat = torch.arange(512, dtype=torch.int32)
+    for replaced in ((), ("table",), ("ctl", "nblocks"), tuple(views)):
+        meta = torch.zeros(512, dtype=torch.int32)
+        parts = {n: meta[at: at + size].view(shape) for n, (at, size, shape) in views.items()}
+        st = LayerStorage(*[None] * 8, meta=meta, **parts)
+        for name in replaced:
+            setattr(st, name, torch.zeros_like(parts[name]))
+        st.load(flat, views)
+        for name, (at, size, shape) in views.items():
+            assert torch.equal(getattr(st, name), flat[at: at + size].view(shape)), (replaced, name)
+    bare = LayerStorage(*[None] * 8, **{n: torch.zeros(shape, dtype=torch.int32) for n, (_, _, shape) in views.items()})
+    bare.load(flat, views)
+    assert torch.equal(bare.warm_free, flat[384:389])
