@@ -6,7 +6,7 @@
 //
 // Fast path (block_size 16, head_dim 64 or 128, GQA group <= 16), one kernel
 // (a second one finalises the score sums of split launches):
-//   * workgroup = (sequence, kv head, split), 4 or 8 waves (plan_cost; 4 when
+//   * workgroup = (sequence, kv head, split), 4 or 8 waves (decode_plan.h; 4 when
 //     the GQA group exceeds 8); the whole GQA group is served by one pass over
 //     each K/V byte; unsplit launches of a batch that is a multiple of 8 place each
 //     sequence's kv heads on one XCD;

@@ -34,7 +34,7 @@
 // two-pass kernel whose four waves took 16 queries each and walked all of K
 // together (B x tokens, 32 / 8 heads, D = 128, fp16): 16 x 2048 700 -> 370 us,
 // 16 x 700 134 -> 55, 2 x 300 41 -> 12, 2 x 4096 453 -> 202, 1 x 8192 (two
-// passes) 746 -> 560; 3 x 1001, 32 / 4 heads, D = 64, bf16 163 -> 20 (that
+// passes) 746 -> 560; 3 x 1001, 32 / 4 heads, D = 64, bf16 163 -> 18.8 (that
 // kernel ran 192 workgroups there, each a chain of 63 tiles, twice, for 8
 // heads).  Splitting the keys needs no barrier per tile and gives every wave
 // the same number of tiles; eight waves per workgroup at 2048 tokens took
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(RED_COLS * RED_ROWS) void prefill_mass_reduce_kerne
 // The two head sets of a group above four heads run side by side, each
 // workgroup half as long, when the launch has no more than eight rows per CU
 // (and the workspace holds a partial row for each): 1 x 1000 (8 / 1 heads,
-// D = 128) 22.1 -> 14.4 us, 3 x 1001 (32 / 4, D = 64) 21.6 -> 19.0,
+// D = 128) 22.1 -> 14.4 us, 3 x 1001 (32 / 4, D = 64) 21.6 -> 18.8,
 // 4 x 2048 (32 / 4, D = 128) 99.7 -> 97.7, 1 x 8192 626 -> 585.  Longer
 // launches are full either way and read twice the partials: 16 x 700
 // (32 / 4, D = 64, 2816 rows) 41.7 -> 42.8, 2 x 4096 (64 / 8, D = 128, 4096
