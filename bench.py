@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Tiered paged decode-attention benchmark on one MI355X.
 
-Workload (the metric's config): Llama-3-8B shape,
+Workload (C3, the metric's configuration): Llama-3-8B shape,
 32 query / 8 KV heads, head_dim 128, batch 32, 4096-token contexts (256
 blocks of 16), per sequence 26 HOT fp16 / 154 WARM int8-absmax / 76 COLD
 (masked) blocks, slots shuffled across shared pools.  One step = one
@@ -49,10 +49,10 @@ def parse():
                    help="c2a / promote / c2b: demotion / promotion / scoring microbenchmarks, c5: end-to-end random-init "
                         "Llama-3-8B decode through the HF hooks (each its own JSON line)")
     p.add_argument("--warm-format", choices=["absmax_i8", "ref_u8"], default="absmax_i8",
-                   help="c3 / c4 / c2a / promote: WARM codec (BASELINE's int8 absmax, or the reference's uint8 "
+                   help="c3 / c4 / c2a / promote: WARM codec (int8 absmax, or the reference's uint8 "
                         "per-token)")
     p.add_argument("--cold", choices=["masked", "zero_logit"], default="masked",
-                   help="c3 / c4: COLD semantics (BASELINE's masked eviction, or the reference's zero-logit tokens)")
+                   help="c3 / c4: COLD semantics (masked eviction, or the reference's zero-logit tokens)")
     p.add_argument("--scores", action="store_true",
                    help="c3 / c4: the policy-step launch that also returns per-block probability sums")
     p.add_argument("--c5-steps", type=int, default=256)
@@ -80,7 +80,7 @@ def parse():
 def build_layers(args, device):
     """``--layers`` distinct layer buffers of the C3 / C4 workload, generated
     on the GPU from seeded generators; WARM tiles quantized on the GPU into
-    the ``--warm-format`` pools (BASELINE's int8 absmax, or the reference's
+    the ``--warm-format`` pools (int8 absmax, or the reference's
     uint8 per-token codec)."""
     import torch
 
@@ -356,7 +356,7 @@ C1_METRIC = "tiered decode-attn µs per launch, TinyLlama shape, batch 1, 512-to
 
 
 def run_c1(args, device):
-    """TinyLlama shape (32 q / 4 kv heads, head_dim
+    """C1: TinyLlama shape (32 q / 4 kv heads, head_dim
     64), batch 1, 512-token context: 8 HOT fp16 / 16 WARM int8-absmax / 8 COLD
     (masked) blocks in a dense pool of 64 blocks (physical ids shuffled).  It
     moves 271 KB, so a launch is latency-bound: the value is the time of one
@@ -517,12 +517,12 @@ C2B_METRIC = "block-score + tier-label µs per call, probs [32, 32, 4096] -> per
 
 
 def run_c2a(args, device):
-    """BASELINE.json configs[1](a): quantize a seeded 50 % of a 4096-block
+    """C2(a): quantize a seeded 50 % of a 4096-block
     fp16 pool (8 kv heads, 16 x 128) into WARM slots, table/state rewrite
     fused.  One step = one launch; 3 source pools are rotated (805 MB).
 
     ``--warm-format`` picks the codec: int8 absmax with fp32 per-(block,
-    head) scales (BASELINE's), or the reference's uint8 with fp16 per-token
+    head) scales, or the reference's uint8 with fp16 per-token
     scale and zero point (quantize_fp16_to_int8, tierkv_policy.py:21-36).
     ``--workload promote`` times the way back (promote_to_hot,
     tierkv_policy.py:1087-1115): the same 2048 blocks dequantized from 3
@@ -642,7 +642,7 @@ def run_c2a(args, device):
 
 
 def run_c2b(args, device):
-    """BASELINE.json configs[1](b): per-block probability mass of fp32
+    """C2(b): per-block probability mass of fp32
     probabilities [32, 32, 4096] and top-k HOT / bottom-k COLD tier labels
     (26 HOT incl. blocks 0 and 255, 77 COLD).  One step = the block-mass
     launch plus the label launch; 20 probability buffers are rotated
@@ -890,7 +890,7 @@ def run_microbench(args, device):
 
 
 def run_ref(args, device):
-    """The reference's end-to-end setting through this build's drop-in for
+    """The reference's end-to-end setting through the drop-in for
     its Python API: a random-init TinyLlama-1.1B-shaped model (22 layers,
     hidden 2048, 32 / 4 heads, head_dim 64, FFN 5632, vocab 32000, fp16),
     batch 1, a uniform-random prompt, greedy decode through the HF hooks and

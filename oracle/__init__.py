@@ -19,7 +19,7 @@ it follows.  Modules:
 * ``block_manager`` -- the native BlockManager's allocation/state rules.
 * ``runtime``       -- the batched runtime's allocation order and tick rules
                        (per-sequence rules of the reference runtime; the
-                       batch-level order is this build's own).
+                       batch-level order has no counterpart there).
 
 The reference-API pools and runtime (paged_tierkv_amd.tierkv_policy) have no
 restatement here: they are pinned directly against trajectories the

@@ -19,7 +19,7 @@ Two formats:
    Pinned by golden vectors written from the reference function itself
    (tests/golden/make_golden.py) and by closed-form special cases.
 
-2. Block absmax format (the reference has no symmetric
+2. Block absmax format (the benchmark configurations; the reference has no symmetric
    quantizer).  Per (block, kv head) over block_size x head_dim:
 
        s = fp32(max|x|) / 127      (IEEE fp32 division)

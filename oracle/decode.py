@@ -14,8 +14,8 @@ and two COLD semantics the HIP path supports:
 * COLD block, ``zero_logit`` (reference): K = V = 0 for the block's valid
   tokens, which still enter the softmax with logit 0
   (tierkv_triton.py:92-102 masked loads -> 0; eager 768-774).
-  COLD block, ``masked``: the block contributes no tokens (
-  "cold evicted (masked out)").
+  COLD block, ``masked``: the block contributes no tokens (the benchmark
+  configurations' "cold evicted (masked out)").
 * Tokens ``t >= block_lengths[b]`` are invalid (tierkv_triton.py:104-106, 777).
 * GQA: q head ``h`` reads kv head ``h // groups`` (tierkv_triton.py:71, 790-792).
 * Softmax in float64 over all valid tokens; an all-invalid row gives 0

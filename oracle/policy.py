@@ -14,7 +14,7 @@
 * ``desired_prefill_states`` restates TieredKVRuntime._desired_prefill_states
   (tierkv_policy.py:1695-1720).
 * ``block_mass_from_probs`` / ``block_mass_from_sums`` define the HIP
-  block-score kernels' fixed reduction order (BASELINE config 2(b)):
+  block-score kernels' fixed reduction order (workload C2(b)):
   per token a sequential fp32 sum over heads h = 0..H-1, then a pairwise
   tree over the block's tokens ((t0+t1)+(t2+t3))+..., then ``/ H`` and
   ``/ max(len, 1)`` (two IEEE fp32 divisions).  The reference's own mean is

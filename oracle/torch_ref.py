@@ -18,7 +18,7 @@ times it, ``tests/test_oracle_torch_ref.py`` checks it against
 * a batch is served as a loop over sequences, one batch-1 call each, as the
   reference serves concurrent requests (main.py:1182-1189).
 
-In the ``masked`` COLD mode (BASELINE's "evicted, masked out") a COLD block's
+In the ``masked`` COLD mode ("evicted, masked out") a COLD block's
 tokens are invalid instead of zero-logit.
 
 ``vectorized_decode`` computes the same quantity for the whole batch with

@@ -6,7 +6,7 @@ Modules:
                     tierkv_policy)
   block_manager  -- BlockManager over the native C++ implementation
   kernels        -- demotion / promotion / block-score / label kernels
-  workloads      -- seeded BASELINE configurations
+  workloads      -- seeded benchmark configurations
   build          -- builds libtierkv_hip.so for gfx950
 """
 

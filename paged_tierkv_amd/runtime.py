@@ -19,7 +19,7 @@ resident on the device:
   steps runs ``tierkv_runtime_tick`` (scores -> labels -> migrations on the
   device).  The host never waits for the device inside a step.
 
-Budgets are fractions of each sequence's current block count (BASELINE's
+Budgets are fractions of each sequence's current block count (workload
 C5: 15 % HOT, 55 % WARM, the rest evicted), evaluated on the host from the
 lockstep block count.
 """

@@ -1,4 +1,4 @@
-"""Seeded synthetic inputs for the BASELINE configurations.
+"""Seeded synthetic inputs for the benchmark configurations.
 
 Every tensor is generated on the CPU with a seeded ``torch.Generator`` so
 the HIP path and the CPU oracle see identical bits; callers move what they
@@ -6,7 +6,7 @@ need to the GPU.  WARM tiles are returned as fp16 *sources*
 (``warm_src_k/v``); the caller quantizes them (the HIP demotion kernel on the
 GPU, or the oracle codec on the CPU).
 
-Configs (BASELINE.json ``configs``):
+Configurations:
 
 * C1 -- TinyLlama shape: 32 q / 4 kv heads, head_dim 64, batch 1, 512
   tokens = 32 blocks of 16; 8 HOT / 16 WARM / 8 COLD; block 0 always HOT,
@@ -281,7 +281,7 @@ C2B_WARM_BUDGET = 256 - C2B_HOT_BUDGET - C2B_COLD_COUNT
 
 
 def llama3_8b_random(device, num_layers: int = 32):
-    """Random-init Llama-3-8B-shaped decoder:
+    """Random-init Llama-3-8B-shaped decoder (workload C5):
     32 layers, hidden 4096, 32 / 8 heads, head_dim 128, FFN 14336, vocab
     128256, fp16 weights ~N(0, 0.02) (transformers' own init with
     initializer_range 0.02), built directly on ``device``."""

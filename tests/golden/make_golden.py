@@ -46,7 +46,7 @@ REF_BM_DIR = os.path.join(os.path.dirname(os.path.dirname(HERE)), "oracle", "_re
 # code path exercised).
 TRAJ = dict(num_layers=2, kv_heads=2, head_dim=16, block_size=16, heads=4, hot_budget=4, warm_budget=3,
             max_seq_len=320, policy_interval=4, pool_chunk_blocks=16, prefill_tokens=90, steps=40)
-# TinyLlama-1.1B's attention geometry, shorter run.
+# TinyLlama-1.1B's attention geometry (workload C1), shorter run.
 TRAJ_TINYLLAMA = dict(TRAJ, kv_heads=4, head_dim=64, heads=32, prefill_tokens=72, steps=24)
 POOL_NAMES = ("hot_k_pool", "hot_v_pool", "warm_k_pool", "warm_v_pool", "k_scale", "k_zero", "v_scale", "v_zero")
 

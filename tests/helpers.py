@@ -9,7 +9,7 @@ import torch
 from oracle import codec
 from oracle import decode as odecode
 
-ATOL = 2e-3   # BASELINE.json north_star tolerance vs the fp32 reference
+ATOL = 2e-3   # parity tolerance vs the fp32 reference
 RTOL = 1e-2
 
 

@@ -1,4 +1,4 @@
-"""BASELINE configs[4] (C5) end to end on the GPU, at its full shape.
+"""Workload C5 end to end on the GPU, at its full shape.
 
 Random-init Llama-3-8B (32 layers, hidden 4096, 32 / 8 heads, head_dim 128,
 FFN 14336, vocab 128256, fp16), batch 16, a 2048-token uniform-random prompt,

@@ -1,7 +1,7 @@
 """GPU parity of the tiered decode-attention kernels against the CPU oracle
 (oracle.decode restates _eager_reference_decode, tierkv_triton.py:708-820).
 
-Tolerance: BASELINE's 2e-3 absolute / 1e-2 relative vs the fp32 reference
+Tolerance: 2e-3 absolute / 1e-2 relative vs the fp32 reference
 for outputs; the same for per-block probability sums."""
 
 from __future__ import annotations
@@ -45,7 +45,7 @@ def _check(case, fmt, device, cold_mode=None, return_scores=False, seqs=None, qu
     return out, scores
 
 
-# -- BASELINE configs -------------------------------------------------------
+# -- benchmark configurations ------------------------------------------------
 
 def test_c1_absmax_masked(device):
     _check(W.config1(), "absmax_i8", device, return_scores=True)

@@ -19,7 +19,7 @@ block_scores_from_probability_sums is fp32 arithmetic whose reduction order
 the reference leaves to ATen: compared within 1e-6 relative.  Finally the
 decode kernel runs over the replayed tables through the reference's calling
 convention (modeling_llama.py:433-456) and is compared with fp32 attention
-over the reconstructed K/V, within the BASELINE tolerance."""
+over the reconstructed K/V, within the parity tolerance."""
 
 from __future__ import annotations
 

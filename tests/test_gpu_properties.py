@@ -6,7 +6,7 @@ both COLD modes, score sums on or off, automatic or forced splits, and the
 default or the deterministic tile hand-out (two launches, the same bits); and
 rows of the long-row list build (513 to 2600 blocks) at many split counts.
 
-Tolerance: BASELINE's 2e-3 absolute / 1e-2 relative vs the fp32 oracle for
+Tolerance: 2e-3 absolute / 1e-2 relative vs the fp32 oracle for
 outputs and per-block probability sums (the same bar as test_gpu_decode)."""
 
 from __future__ import annotations

@@ -10,7 +10,7 @@ other GPU tests:
   fp16 maximum (a row whose range overflows to infinity takes the IEEE
   path).  Codes, scales, zero points and the promoted fp16 values bit for
   bit (quantize_fp16_to_int8 / dequantize_int8_to_fp16,
-  tierkv_policy.py:21-44; BASELINE's absmax codec);
+  tierkv_policy.py:21-44; the absmax codec);
 * block mass from probabilities (bit for bit) and tier labels (exactly) over
   random shapes, block sizes, lengths, budgets, modes and score ties
   (compute_block_scores, tierkv_policy.py:1380-1389; enforce_budget /
@@ -19,7 +19,7 @@ other GPU tests:
   dim, prompt length from one token, steps, tick interval, budgets, policy
   mode, WARM format, COLD mode): tables, states, lengths and pool contents
   equal to oracle.runtime after the prefill and after every step, decode
-  outputs within BASELINE's tolerance (the runtime generalises
+  outputs within the parity tolerance (the runtime generalises
   TieredKVRuntime, tierkv_policy.py:1534-1912, to a batch);
 * prefill block scores over random batch, GQA group (1-8), prompt length,
   head dim, block size, dtype and logit scale, at 1e-4 relative to the

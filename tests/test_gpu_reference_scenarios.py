@@ -1,4 +1,4 @@
-"""The reference's own runtime-level tests, run against this build's drop-in
+"""The reference's own runtime-level tests, run against the drop-in
 for its Python API (paged_tierkv_amd.tierkv_policy + BlockManager), with
 the reference's inputs and assertions:
 

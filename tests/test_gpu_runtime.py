@@ -6,7 +6,7 @@ Bit-exact: slot tables, states, lengths, block counts, HOT contents and WARM
 codes / scales of every live block (the allocation order is fixed).  The
 tick ranks the decode kernel's own probability sums on both sides, so the
 label decisions are compared on identical inputs.  Attention outputs: the
-BASELINE tolerance (2e-3 abs, 1e-2 rel) against the oracle decode over the
+parity tolerance (2e-3 abs, 1e-2 rel) against the oracle decode over the
 oracle's pools."""
 
 from __future__ import annotations

@@ -1,6 +1,6 @@
 """Pins for the oracle decode (CPU): textbook attention on all-HOT inputs
 (torch SDPA in fp32), closed-form COLD identities, GQA/MHA equivalence, the
-reference's score normalisation, and the BASELINE ideal-byte figures."""
+reference's score normalisation, and the benchmark ideal-byte figures."""
 
 from __future__ import annotations
 

@@ -9,7 +9,7 @@ and lengths must equal the reference's BlockManager states and length table
 exactly.  Ticks take the recorded block scores directly (the block mass of
 probability sums is pinned on its own by closed forms).
 
-Slot ids of a batch are this build's own allocation order (the reference has
+Slot ids of a batch follow an allocation order of their own (the reference has
 no batch); they are checked by invariants: every resident block owns a
 distinct slot of its tier, and free stacks plus owned slots cover every slot
 exactly once."""
