@@ -30,6 +30,8 @@ constexpr int STAGE_GLOBAL = 0;
 constexpr int STAGE_LDS_BLOCK = 1;
 constexpr int STAGE_LDS_LIST = 2;
 constexpr int MAX_SPLIT_UNITS = 1 << 16;   // units per launch when a unit is split
+constexpr int CUS = 256;           // compute units of the GPU, 32 in each of 8 XCDs
+constexpr int CU_LDS = 160 * 1024; // bytes of LDS per compute unit
 
 struct Plan {
   int nw;
@@ -89,15 +91,14 @@ inline int waves_per_simd(int head_dim, int warm_format, bool scores) {
   return warm_format == TIERKV_WARM_ABSMAX_I8 && !scores ? 4 : 3;
 }
 
-// Workgroups of nw waves that run together on a CU (four SIMDs, 160 KB of
-// LDS).  A score launch of a large group at head_dim 64 is held to fewer by
+// Workgroups of nw waves that run together on a CU (four SIMDs).  A score launch of a large group at head_dim 64 is held to fewer by
 // its statistics than by registers.
 inline int64_t workgroups_per_cu(int num_blocks, int groups, int head_dim, int warm_format, bool scores, int nw,
                                  int s) {
   const int64_t by_registers = 4 * waves_per_simd(head_dim, warm_format, scores) / nw;
   const int64_t lds = STATIC_LDS + dynamic_lds(nw, groups, head_dim, num_blocks,
                                                score_stage(scores, groups, num_blocks, s));
-  return std::max<int64_t>(1, std::min(by_registers, 160 * 1024 / lds));
+  return std::max<int64_t>(1, std::min(by_registers, CU_LDS / lds));
 }
 
 // Expected time (us, less the launch itself) of a launch with nw waves per
@@ -126,7 +127,7 @@ inline double plan_cost(int64_t units, int num_blocks, int groups, int head_dim,
   const double alone = head_dim == 64 && nw == 4 ? 1.42 : 1.0;
   const double fixed = nw == 4 ? 3.98 : 5.17;
   const int64_t room = workgroups_per_cu(num_blocks, groups, head_dim, warm_format, scores, nw, s);
-  const int64_t on_cu = (units * s + 255) / 256;
+  const int64_t on_cu = (units * s + CUS - 1) / CUS;
   const int64_t passes = (on_cu + room - 1) / room;
   const double refill = room == 1 ? 1.44 : nw == 4 ? 1.81 : 1.21;   // a further pass's fixed part against the first's
   auto pass = [&](int64_t together) { return per_block * num_blocks / s * std::max(double(together), alone); };
