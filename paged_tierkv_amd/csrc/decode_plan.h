@@ -112,37 +112,37 @@ inline int64_t workgroups_per_cu(int num_blocks, int groups, int head_dim, int w
 // 16, both head dims and formats, with and without score sums, 5 to 30 % HOT
 // and 40 to 65 % WARM, each with both wave counts and up to 13 split counts,
 // in graphs over four layers' buffers.  The plan chosen by it is on average
-// 0.6 % slower than the fastest measured one (fitted on either half and
-// checked on the other, too); the plain rule of required_splits with the most
+// 0.6 % slower than the fastest measured one, also over 1,200 further shapes
+// that the fit has not seen; the plain rule of required_splits with the most
 // waves is 15 % slower, up to 3.5 times (units * s just above what runs at
-// once).  1 shape in 50 is more than 3 % slower than with it (worst
-// 1.14 times).
+// once).  1 shape in 60 is more than 3 % slower than with it (worst
+// 1.12 times).
 inline double plan_cost(int64_t units, int num_blocks, int groups, int head_dim, int warm_format, bool scores, int nw,
                         int s) {
   // A block's tiles in a workgroup, alone or sharing its CU: 256 units, D =
   // 128, 10 % HOT, 60 % WARM (3.3 KB per block) take 25.6 us at 144 blocks and
-  // 58.3 at 400, 0.128 per block (26 B/ns).  Four waves alone at D = 64 have
-  // too few loads in flight (64 units of 256 blocks: 25.1 us, 18.6 with eight).
-  const double per_block = head_dim == 64 ? 0.060 : 0.125;
-  const double alone = head_dim == 64 && nw == 4 ? 1.42 : 1.0;
-  const double fixed = nw == 4 ? 3.98 : 5.17;
+  // 58.3 at 400, 0.128 per block (26 B/ns; smaller launches are served by the
+  // caches in part).  Four waves alone at D = 64 have too few loads in flight
+  // (64 units of 256 blocks: 25.1 us, 18.6 with eight).
+  const double per_block = head_dim == 64 ? 0.063 : 0.117;
+  const double alone = head_dim == 64 && nw == 4 ? 1.38 : 1.0;
+  const double fixed = head_dim == 64 ? (nw == 4 ? 4.19 : 4.97) : (nw == 4 ? 5.07 : 5.94);
   const int64_t room = workgroups_per_cu(num_blocks, groups, head_dim, warm_format, scores, nw, s);
   const int64_t on_cu = (units * s + CUS - 1) / CUS;
   const int64_t passes = (on_cu + room - 1) / room;
-  const double refill = room == 1 ? 1.44 : nw == 4 ? 1.81 : 1.21;   // a further pass's fixed part against the first's
+  const double refill = nw == 4 && room > 1 ? 1.48 : 1.3;   // a further pass's fixed part against the first's
   auto pass = [&](int64_t together) { return per_block * num_blocks / s * std::max(double(together), alone); };
   double t = fixed + (passes - 1) * (fixed * refill + pass(std::min(on_cu, room))) +
              pass(on_cu - (passes - 1) * room);
-  const int threads = 64 * nw, elements = groups * head_dim;
   if (s > 1) {
-    // Publication and merge: MERGE_UNROLL splits and one or two elements per
-    // thread and round trip; workgroups on one CU publish in turn (64 units of
-    // 256 blocks, D = 64, G = 4: 14.5 us in two splits of eight waves, 12.0 in
-    // four, 14.7 in five, where two share a CU).
+    // Publication and merge, by the unit's elements and MERGE_UNROLL splits
+    // per round trip (in four splits instead of one, four waves, under 48
+    // blocks, D = 128: 0.1 us more with four heads, 0.7 with eight, 4.3 with
+    // sixteen); workgroups on one CU publish in turn (64 units of 256 blocks,
+    // D = 64, G = 4: 14.5 us in two splits of eight waves, 12.0 in four, 14.7
+    // in five, where two share a CU).
     const int rounds = (s + MERGE_UNROLL - 1) / MERGE_UNROLL;
-    const int per_trip = elements > threads ? 2 * threads : threads;
-    t += 0.59 * rounds + 0.96 * rounds * ((elements + per_trip - 1) / per_trip) +
-         0.61 * ((elements + threads - 1) / threads) + 1.52 * (std::min(on_cu, room) - 1);
+    t += 0.95 * rounds + (0.57 + 0.89 * rounds) * (groups * head_dim / 512.0) + 1.59 * (std::min(on_cu, room) - 1);
   }
   // Score sums: the workgroup's own waves, a head or a part of one each (8
   // units of 64 blocks unsplit, G = 4: 10.9 -> 13.8 us with eight waves, 11.5
@@ -150,16 +150,17 @@ inline double plan_cost(int64_t units, int num_blocks, int groups, int head_dim,
   // head) row (the same in eight splits 8.8 -> 13.4 us; 1024 rows, 128 units
   // of 256 blocks at D = 64 in two splits: 29.7 us, 23.2 unsplit).
   if (scores && score_stage(scores, groups, num_blocks, s) == STAGE_LDS_BLOCK)
-    t += 1.9 * (((groups <= 8 ? 8 / groups * groups : groups) + nw - 1) / nw);
+    t += 1.7 * (((groups <= 8 ? 8 / groups * groups : groups) + nw - 1) / nw);
   else if (scores)
-    t += 4.27 + 5.06 * double(units * groups) / 512;
+    t += 4.22 + 5.05 * double(units * groups) / 512;
   // The list build of rows beyond one chunk (256 units, D = 128, four waves
   // against eight: 0.5 us less at 256 blocks, 0.6 more at 320), and beyond one
   // pass (32 units of 2048 blocks in eight splits: 30.7 us with eight waves,
   // one pass; 32.1 with four, two), where the blanks of the score sums are
   // written one by one.
-  if (num_blocks > threads) t += 1.09;
-  t += ((num_blocks - 1) / (PRE_CHUNKS * threads)) * (scores ? 4.9 : 1.5);
+  const int threads = 64 * nw;
+  if (num_blocks > threads) t += 1.17;
+  t += ((num_blocks - 1) / (PRE_CHUNKS * threads)) * (scores ? 5.28 : 1.5);
   return t;
 }
 
@@ -211,7 +212,9 @@ inline int64_t least_workspace(int batch, int num_heads, int kv_heads, int num_b
 // Wave and split counts of a fast-path launch: the cheapest by plan_cost whose
 // workspace fits workspace_bytes (that of required_splits always does); a
 // split hint fixes the splits.  GQA groups above 8 take four waves, to bound
-// the LDS accumulators.
+// the LDS accumulators.  Another plan has to promise 2 % over the plain rule's
+// (its splits with the most waves): of 2,536 shapes those then measured more
+// than 3 % slower than it fall from 54 to 43, the mean stays.
 // The plan decides in which groups a deterministic launch adds its partial
 // sums, so its output's bits are the plan's: such a launch takes the free plan
 // in every workspace with room for it, and in every smaller one the plan of
@@ -224,12 +227,15 @@ inline Plan plan_launch(int batch, int num_heads, int kv_heads, int num_blocks, 
     return ws_layout(batch, num_heads, kv_heads, num_blocks, block_size, head_dim, scores, s).total;
   };
   auto cheapest = [&](int64_t room) -> Plan {
-    Plan best{4, required_splits(units, num_blocks, groups, splits_hint)};
-    double best_cost = 1e300;
+    Plan best{groups <= 8 ? 8 : 4, required_splits(units, num_blocks, groups, splits_hint)};
+    auto cost = [&](int nw, int s) {
+      return plan_cost(units, num_blocks, groups, head_dim, warm_format, scores, nw, s);
+    };
+    double best_cost = cost(best.nw, best.splits) / 1.02;
     auto consider = [&](int s) {
       for (int nw = 8; nw >= 4; nw -= 4) {
         if (nw == 8 && groups > 8) continue;
-        const double c = plan_cost(units, num_blocks, groups, head_dim, warm_format, scores, nw, s);
+        const double c = cost(nw, s);
         if (c < best_cost) {
           best_cost = c;
           best = Plan{nw, s};

@@ -534,8 +534,8 @@ def test_workspace_reuse_across_shapes(device):
 @pytest.mark.parametrize("batch,kv,groups,dim,nb,lens,fmt", [
     (1, 4, 4, 128, 9, False, "absmax_i8"),     # four waves (eight with score sums), about one tile each
     (2, 8, 4, 128, 64, True, "ref_u8"),        # four waves, eight splits: two output elements per merging thread
-    (1, 4, 3, 64, 400, True, "ref_u8"),        # eight waves, eight splits; 192 elements in a 512-thread merge
-    (2, 2, 8, 128, 150, False, "absmax_i8"),   # eight waves, eight splits, 1024 elements per unit
+    (1, 4, 3, 64, 400, True, "ref_u8"),        # eight waves, sixteen splits; 192 elements in a 512-thread merge
+    (2, 2, 8, 128, 150, False, "absmax_i8"),   # four waves, eight splits, 1024 elements per unit
     (31, 8, 1, 64, 20, True, "absmax_i8"),     # 248 units, unsplit; one head per unit
     (40, 8, 2, 64, 33, True, "ref_u8"),        # more units than CUs
     (1, 1, 16, 128, 300, True, "ref_u8"),      # sixteen heads: four waves, eight elements per merging thread
